@@ -19,6 +19,7 @@
 
 #include "ostc_fr.hpp"
 #include "ostc_inflow.hpp"
+#include "ostc_weno.hpp"
 
 namespace ostc {
 namespace fr {
@@ -31,98 +32,6 @@ __device__ __forceinline__ long long pid(const FrBlockDev& B, int i, int j, int 
 }
 __device__ __forceinline__ long long pid0(const FrBlockDev& B, int i, int j, int k) {
   return ((long long)k * B.my + j) * B.mx + i;
-}
-
-// WENO-Z5, src/WENO.cu:1582-1617
-__device__ __forceinline__ double weno5z(const double* vp, const double* vm, double eps) {
-  constexpr double one6th{1.0 / 6};
-  double v0{one6th * (2 * vp[2] + 5 * vp[3] - vp[4])};
-  double v1{one6th * (-vp[1] + 5 * vp[2] + 2 * vp[3])};
-  double v2{one6th * (2 * vp[0] - 7 * vp[1] + 11 * vp[2])};
-  constexpr double c1312{13.0 / 12};
-  double b0 = c1312 * (vp[2] + vp[4] - 2 * vp[3]) * (vp[2] + vp[4] - 2 * vp[3]) +
-              0.25 * (3 * vp[2] - 4 * vp[3] + vp[4]) * (3 * vp[2] - 4 * vp[3] + vp[4]);
-  double b1 = c1312 * (vp[1] + vp[3] - 2 * vp[2]) * (vp[1] + vp[3] - 2 * vp[2]) +
-              0.25 * (vp[1] - vp[3]) * (vp[1] - vp[3]);
-  double b2 = c1312 * (vp[0] + vp[2] - 2 * vp[1]) * (vp[0] + vp[2] - 2 * vp[1]) +
-              0.25 * (vp[0] - 4 * vp[1] + 3 * vp[2]) * (vp[0] - 4 * vp[1] + 3 * vp[2]);
-  double tau{(b0 - b2) * (b0 - b2)};
-  double a0{0.3 + 0.3 * tau / ((eps + b0) * (eps + b0))};
-  double a1{0.6 + 0.6 * tau / ((eps + b1) * (eps + b1))};
-  double a2{0.1 + 0.1 * tau / ((eps + b2) * (eps + b2))};
-  const double fp{(a0 * v0 + a1 * v1 + a2 * v2) / (a0 + a1 + a2)};
-  v0 = one6th * (11 * vm[2] - 7 * vm[3] + 2 * vm[4]);
-  v1 = one6th * (2 * vm[1] + 5 * vm[2] - vm[3]);
-  v2 = one6th * (-vm[0] + 5 * vm[1] + 2 * vm[2]);
-  b0 = c1312 * (vm[2] + vm[4] - 2 * vm[3]) * (vm[2] + vm[4] - 2 * vm[3]) +
-       0.25 * (3 * vm[2] - 4 * vm[3] + vm[4]) * (3 * vm[2] - 4 * vm[3] + vm[4]);
-  b1 = c1312 * (vm[1] + vm[3] - 2 * vm[2]) * (vm[1] + vm[3] - 2 * vm[2]) + 0.25 * (vm[1] - vm[3]) * (vm[1] - vm[3]);
-  b2 = c1312 * (vm[0] + vm[2] - 2 * vm[1]) * (vm[0] + vm[2] - 2 * vm[1]) +
-       0.25 * (vm[0] - 4 * vm[1] + 3 * vm[2]) * (vm[0] - 4 * vm[1] + 3 * vm[2]);
-  tau = (b0 - b2) * (b0 - b2);
-  a0 = 0.1 + 0.1 * tau / ((eps + b0) * (eps + b0));
-  a1 = 0.6 + 0.6 * tau / ((eps + b1) * (eps + b1));
-  a2 = 0.3 + 0.3 * tau / ((eps + b2) * (eps + b2));
-  const double fm{(a0 * v0 + a1 * v1 + a2 * v2) / (a0 + a1 + a2)};
-  return fp + fm;
-}
-
-// WENO-Z7, src/WENO.cu:1619-1693.  vp = F+ at i-3..i+3, vm = F- at i-2..i+4.
-__device__ __forceinline__ double weno7z(const double* vp, const double* vm, double eps) {
-  constexpr double one6th{1.0 / 6}, d12{13.0 / 12.0}, d13{1043.0 / 960}, d14{1.0 / 12};
-  constexpr double c0{1.0 / 35}, c1{12.0 / 35}, c2{18.0 / 35}, c3{4.0 / 35}, one12th{1.0 / 12};
-  double s1 = one6th * (-2 * vp[0] + 9 * vp[1] - 18 * vp[2] + 11 * vp[3]);
-  double s2 = -vp[0] + 4 * vp[1] - 5 * vp[2] + 2 * vp[3];
-  double s3 = -vp[0] + 3 * vp[1] - 3 * vp[2] + vp[3];
-  double b0 = s1 * s1 + d12 * s2 * s2 + d13 * s3 * s3 + d14 * s1 * s3;
-  s1 = one6th * (vp[1] - 6 * vp[2] + 3 * vp[3] + 2 * vp[4]);
-  s2 = vp[2] - 2 * vp[3] + vp[4];
-  s3 = -vp[1] + 3 * vp[2] - 3 * vp[3] + vp[4];
-  double b1 = s1 * s1 + d12 * s2 * s2 + d13 * s3 * s3 + d14 * s1 * s3;
-  s1 = one6th * (-2 * vp[2] - 3 * vp[3] + 6 * vp[4] - vp[5]);
-  s3 = -vp[2] + 3 * vp[3] - 3 * vp[4] + vp[5];
-  double b2 = s1 * s1 + d12 * s2 * s2 + d13 * s3 * s3 + d14 * s1 * s3;
-  s1 = one6th * (-11 * vp[3] + 18 * vp[4] - 9 * vp[5] + 2 * vp[6]);
-  s2 = 2 * vp[3] - 5 * vp[4] + 4 * vp[5] - vp[6];
-  s3 = -vp[3] + 3 * vp[4] - 3 * vp[5] + vp[6];
-  double b3 = s1 * s1 + d12 * s2 * s2 + d13 * s3 * s3 + d14 * s1 * s3;
-  double tau = (b0 - b3) * (b0 - b3);
-  double a0 = c0 + c0 * tau / ((eps + b0) * (eps + b0));
-  double a1 = c1 + c1 * tau / ((eps + b1) * (eps + b1));
-  double a2 = c2 + c2 * tau / ((eps + b2) * (eps + b2));
-  double a3 = c3 + c3 * tau / ((eps + b3) * (eps + b3));
-  double v0 = one12th * (-3 * vp[0] + 13 * vp[1] - 23 * vp[2] + 25 * vp[3]);
-  double v1 = one12th * (vp[1] - 5 * vp[2] + 13 * vp[3] + 3 * vp[4]);
-  double v2 = one12th * (-vp[2] + 7 * vp[3] + 7 * vp[4] - vp[5]);
-  double v3 = one12th * (3 * vp[3] + 13 * vp[4] - 5 * vp[5] + vp[6]);
-  const double fp = (a0 * v0 + a1 * v1 + a2 * v2 + a3 * v3) / (a0 + a1 + a2 + a3);
-
-  s1 = one6th * (-2 * vm[6] + 9 * vm[5] - 18 * vm[4] + 11 * vm[3]);
-  s2 = -vm[6] + 4 * vm[5] - 5 * vm[4] + 2 * vm[3];
-  s3 = -vm[6] + 3 * vm[5] - 3 * vm[4] + vm[3];
-  b0 = s1 * s1 + d12 * s2 * s2 + d13 * s3 * s3 + d14 * s1 * s3;
-  s1 = one6th * (vm[5] - 6 * vm[4] + 3 * vm[3] + 2 * vm[2]);
-  s2 = vm[4] - 2 * vm[3] + vm[2];
-  s3 = -vm[5] + 3 * vm[4] - 3 * vm[3] + vm[2];
-  b1 = s1 * s1 + d12 * s2 * s2 + d13 * s3 * s3 + d14 * s1 * s3;
-  s1 = one6th * (-2 * vm[4] - 3 * vm[3] + 6 * vm[2] - vm[1]);
-  s3 = -vm[4] + 3 * vm[3] - 3 * vm[2] + vm[1];
-  b2 = s1 * s1 + d12 * s2 * s2 + d13 * s3 * s3 + d14 * s1 * s3;
-  s1 = one6th * (-11 * vm[3] + 18 * vm[2] - 9 * vm[1] + 2 * vm[0]);
-  s2 = 2 * vm[3] - 5 * vm[2] + 4 * vm[1] - vm[0];
-  s3 = -vm[3] + 3 * vm[2] - 3 * vm[1] + vm[0];
-  b3 = s1 * s1 + d12 * s2 * s2 + d13 * s3 * s3 + d14 * s1 * s3;
-  tau = (b0 - b3) * (b0 - b3);
-  a0 = c0 + c0 * tau / ((eps + b0) * (eps + b0));
-  a1 = c1 + c1 * tau / ((eps + b1) * (eps + b1));
-  a2 = c2 + c2 * tau / ((eps + b2) * (eps + b2));
-  a3 = c3 + c3 * tau / ((eps + b3) * (eps + b3));
-  v0 = one12th * (-3 * vm[6] + 13 * vm[5] - 23 * vm[4] + 25 * vm[3]);
-  v1 = one12th * (vm[5] - 5 * vm[4] + 13 * vm[3] + 3 * vm[2]);
-  v2 = one12th * (-vm[4] + 7 * vm[3] + 7 * vm[2] - vm[1]);
-  v3 = one12th * (3 * vm[3] + 13 * vm[2] - 5 * vm[1] + vm[0]);
-  const double fm = (a0 * v0 + a1 * v1 + a2 * v2 + a3 * v3) / (a0 + a1 + a2 + a3);
-  return fp + fm;
 }
 
 // cv of one point from bv and sv (compute_cv_from_bv_1_point<FR>,
