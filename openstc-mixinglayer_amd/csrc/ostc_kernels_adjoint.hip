@@ -610,49 +610,54 @@ __global__ void k_fourier_grad_final(int n, int n_part, const double* part, doub
   grad[m] = s;
 }
 
-// Row sums S0_j = sum rho, S1_j = sum rho u over i < ni, k < nk.
-__global__ __launch_bounds__(kT) void k_theta_rows(Geo G, const double* cv, int ni, int nk, double* rows) {
-  __shared__ double s0w[kT / 64], s1w[kT / 64];
+// Row sums over i < ni, k < nk: rows[2 j] = sum rho, rows[2 j + 1] = sum rho
+// (u1 - u), coef[2 j + 1] = sum rho (u - u2).  The differences from the streams
+// are summed rather than formed from the mean velocity afterwards: outside the
+// layer one of them vanishes, and a rounded mean velocity would leave
+// 10^-16 u du there, row after row, 3e-15 of theta in all (as much as a change
+// of 10^-6 in the smallest amplitudes; the sums leave a tenth of it).
+__global__ __launch_bounds__(kT) void k_theta_rows(Geo G, const double* cv, ThetaParams T, double* rows, double* coef) {
+  __shared__ double sw[3][kT / 64];
   const int j = blockIdx.x;
-  double a = 0, b = 0;
-  for (long long e = threadIdx.x; e < (long long)ni * nk; e += kT) {
-    const int i = (int)(e % ni), k = (int)(e / ni);
+  double a[3] = {0, 0, 0};
+  for (long long e = threadIdx.x; e < (long long)T.ni * T.nk; e += kT) {
+    const int i = (int)(e % T.ni), k = (int)(e / T.ni);
     const long long p = gidx(G, i, j, k);
-    a += cv[p];
-    b += cv[p + G.sz];
+    const double rho = cv[p], mom = cv[p + G.sz];
+    a[0] += rho;
+    a[1] += __builtin_fma(T.u1, rho, -mom);
+    a[2] += __builtin_fma(-T.u2, rho, mom);
   }
-  a = wave_sum64(a);
-  b = wave_sum64(b);
-  if (threadIdx.x % 64 == 0) {
-    s0w[threadIdx.x / 64] = a;
-    s1w[threadIdx.x / 64] = b;
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    a[q] = wave_sum64(a[q]);
+    if (threadIdx.x % 64 == 0) sw[q][threadIdx.x / 64] = a[q];
   }
   __syncthreads();
   if (threadIdx.x == 0) {
-    double x = 0, y = 0;
-    for (int q = 0; q < kT / 64; ++q) {
-      x += s0w[q];
-      y += s1w[q];
-    }
-    rows[2 * j] = x;
-    rows[2 * j + 1] = y;
+    double x[3] = {0, 0, 0};
+    for (int w = 0; w < kT / 64; ++w)
+      for (int q = 0; q < 3; ++q) x[q] += sw[q][w];
+    rows[2 * j] = x[0];
+    rows[2 * j + 1] = x[1];
+    coef[2 * j + 1] = x[2];
   }
 }
 
-// theta and its derivatives with respect to the row sums (one thread).
+// theta and its derivatives with respect to the row sums of rho and rho u
+// (one thread).
 __global__ void k_theta_final(int my, ThetaParams T, const double* rows, double* coef, double* theta) {
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
   const double N = (double)T.ni * T.nk;
   double th = 0;
   for (int j = 0; j < my; ++j) {
-    const double S0 = rows[2 * j], S1 = rows[2 * j + 1];
-    const double rho = S0 / N, U = S1 / S0;
+    const double S0 = rows[2 * j], d1 = rows[2 * j + 1], d2 = coef[2 * j + 1];
     const double C = ((j == 0 || j == my - 1) ? 0.5 * T.dy : T.dy) / (T.rho0 * T.du * T.du);
-    th += C * rho * (T.u1 - U) * (U - T.u2);
-    const double d_rho = C * (T.u1 - U) * (U - T.u2);
-    const double d_U = C * rho * (T.u1 + T.u2 - 2 * U);
-    coef[2 * j] = d_rho / N - d_U * S1 / (S0 * S0);
-    coef[2 * j + 1] = d_U / S0;
+    const double a = d1 / S0, b = d2 / S0;  // u1 - U, U - u2
+    th += C * (S0 / N) * a * b;
+    // theta_j = C/N (u1 S0 - S1)(S1 - u2 S0) / S0
+    coef[2 * j] = C / N * (T.u1 * b - T.u2 * a - a * b);
+    coef[2 * j + 1] = C / N * (a - b);
   }
   *theta = th;
 }
@@ -741,7 +746,7 @@ void fourier_grad(const DevBlock& B, const FourierModes& F, const double* lam, c
 
 void theta_eval(const DevBlock& B, const ThetaParams& T, const double* cv, double* rows, double* coef, double* theta,
                 hipStream_t st) {
-  k_theta_rows<<<B.my, kT, 0, st>>>(geo_of(B), cv, T.ni, T.nk, rows);
+  k_theta_rows<<<B.my, kT, 0, st>>>(geo_of(B), cv, T, rows, coef);
   k_theta_final<<<1, 64, 0, st>>>(B.my, T, rows, coef, theta);
 }
 
