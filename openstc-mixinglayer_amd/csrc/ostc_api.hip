@@ -107,6 +107,7 @@ struct ostc_ctx_s {
   std::vector<int> plain_comm;
   int tile_index = 0, n_wg = 0, xcd_remap = 1, n_tiles = 0, waves = 0, split = 0;
   int* d_tile_block = nullptr;
+  SweepPlan sweep{};       // work lists of the inviscid sweeps (component-wise WENO schemes)
   double* d_scratch = nullptr;
   int n_first = 1024;
   double* d_dt = nullptr;
@@ -536,6 +537,63 @@ FusedArgs fused_args(ostc_ctx c, int in, int out, int rk) {
   return a;
 }
 
+// Work lists of the inviscid sweeps.  A march is cut where whole columns would
+// leave the chip short of waves (16 per CU wanted: two rounds of the eight its
+// registers admit), down to 4 cells, and at 64 cells, so that no wave is much
+// longer than the others; each cut costs 2 ngg more split points.
+int build_sweeps(ostc_ctx c) {
+  if (!sweep_scheme(c->P.scheme)) return OSTC_OK;
+  std::vector<SweepItem> h[4];
+  for (int d = 0; d < 4; ++d) {
+    if (d == 0 || d == 3) {  // x sweep and viscous kernel: consecutive padded points
+      const int take = d == 0 ? 4 * sweep_valid(c->P.scheme) : visc_cells_per_wg();
+      for (size_t b = 0; b < c->blocks.size(); ++b) {
+        const DevBlock& B = c->blocks[b].d;
+        for (int q = 0; q < B.sx * B.my * B.mz; q += take) h[d].push_back(SweepItem{(int)b, q, 0, 0});
+      }
+    } else {
+      auto columns = [&](const DevBlock& B) { return d == 1 ? B.mx * B.mz : B.mx * B.my; };
+      long long waves = 0;
+      for (auto& B : c->blocks) waves += (columns(B.d) + 63) / 64;
+      const int want = (int)((16LL * c->cus + waves - 1) / waves);
+      for (size_t b = 0; b < c->blocks.size(); ++b) {
+        const DevBlock& B = c->blocks[b].d;
+        const int m = d == 1 ? B.my : B.mz;
+        const int pieces = std::max((m + 63) / 64, std::min(want, (m + 3) / 4));
+        for (int s = 0; s < pieces; ++s) {
+          const int c0 = (int)((long long)m * s / pieces), c1 = (int)((long long)m * (s + 1) / pieces);
+          for (int q = 0; q < columns(B); q += 64) h[d].push_back(SweepItem{(int)b, q, c0, c1 - c0});
+        }
+      }
+    }
+  }
+  std::vector<SweepItem> all;  // one allocation and one copy for the four lists
+  for (auto& l : h) all.insert(all.end(), l.begin(), l.end());
+  void* v = nullptr;
+  HIPCHK(c, hipMalloc(&v, all.size() * sizeof(SweepItem)));
+  c->allocs.push_back(v);
+  HIPCHK(c, hipMemcpy(v, all.data(), all.size() * sizeof(SweepItem), hipMemcpyHostToDevice));
+  size_t at = 0;
+  for (int d = 0; d < 4; ++d) {
+    c->sweep.items[d] = static_cast<SweepItem*>(v) + at;
+    c->sweep.n[d] = (int)h[d].size();
+    at += h[d].size();
+  }
+  return OSTC_OK;
+}
+
+// The kernels of one stage: the sweeps (component-wise schemes) or the tile
+// kernels (characteristic); mode as fused_launch.  False: no kernel for this
+// scheme and tile.
+bool launch_stage(ostc_ctx c, int mode, const FusedArgs& a, long long* n) {
+  if (sweep_scheme(c->P.scheme)) {
+    sweep_launch(a, c->sweep, mode != 1, c->st, n);
+    return true;
+  }
+  ++*n;
+  return fused_launch(c->tile_index, mode, a, c->n_wg, c->st) >= 0;
+}
+
 void launch_group(ostc_ctx c, const Group& g, int slot, int src, long long* n, bool props = false) {
   if (g.hi > g.lo)
     ops_launch(c->d_blocks, (int)c->blocks.size(), c->d_ops, g.lo, g.hi, g.total, slot, src, c->st, n, props);
@@ -699,9 +757,9 @@ int batched_stage(ostc_ctx c, int rk, long long* n, int ev_base) {
   const int in = rk, out = (rk + 1) % kRing;
   FusedArgs a = fused_args(c, in, out, rk);
   if (events) HIPCHK(c, hipEventRecord(c->evpool[ev_base + 2 * rk], c->st));
-  if (fused_launch(c->tile_index, c->split ? 2 : 0, a, c->n_wg, c->st) < 0)
+  if (!launch_stage(c, c->split ? 2 : 0, a, n))
     return fail(c, OSTC_ERR_UNSUPPORTED, "fused kernel: scheme/tile not available");
-  *n += c->split ? 2 : 1;
+  if (c->split && !sweep_scheme(c->P.scheme) && c->P.visc) ++*n;
   if (events) HIPCHK(c, hipEventRecord(c->evpool[ev_base + 2 * rk + 1], c->st));
   const bool fold = c->ghost_props == OSTC_GHOST_PROPS_IN_OPS;
   launch_group(c, c->rim, out, in, n, fold);
@@ -1136,6 +1194,7 @@ int ostc_finalize(ostc_ctx c) {
   c->dq_bar.assign(c->blocks.size(), nullptr);
   c->cv_bar.assign(c->blocks.size(), nullptr);
   if (c->s.fixed_time_step) HIPCHK(c, hipMemcpy(c->d_dt, &c->s.dt, sizeof(double), hipMemcpyHostToDevice));
+  if ((r = build_sweeps(c))) return r;
   c->finalized = true;
   return set_tiles(c, 0, 0);
 }
@@ -1428,7 +1487,8 @@ int ostc_batched_rhs(ostc_ctx c, int b) {
   if ((r = need_fused(c))) return r;
   FusedArgs a = fused_args(c, 0, 1, 0);
   a.target_block = b;
-  if (fused_launch(c->tile_index, 1, a, c->n_wg, c->st) < 0)
+  long long n = 0;
+  if (!launch_stage(c, 1, a, &n))
     return fail(c, OSTC_ERR_UNSUPPORTED, "fused kernel: scheme/tile not available");
   HIPCHK(c, hipGetLastError());
   return OSTC_OK;
@@ -1577,19 +1637,20 @@ int ostc_autotune(ostc_ctx c, int reps, int* best_index, double* best_ms) {
   if (reps < 1) reps = 3;
   double best = 1e30;
   int bi = c->tile_index, bw = 0, bs = 0;
+  long long n = 0;
   const int waves[] = {0, 1, 2, 4};
   for (int idx = 0; idx < fused_shape_count(c->P.scheme); ++idx) {
     const int lds = fused_lds_bytes(c->P.scheme, idx);
     if (lds < 0 || lds > 160 * 1024) continue;
-    for (int sp = 0; sp < (c->P.visc ? 2 : 1); ++sp)
+    for (int sp = 0; sp < (c->P.visc && !sweep_scheme(c->P.scheme) ? 2 : 1); ++sp)
       for (int w : waves) {
         r = ostc_set_tile(c, idx, w, sp);
         if (r) return r;
         FusedArgs a = fused_args(c, 0, 1, 0);
         const int mode = sp ? 2 : 0;
-        if (fused_launch(idx, mode, a, c->n_wg, c->st) < 0) continue;  // warm-up
+        if (!launch_stage(c, mode, a, &n)) continue;  // warm-up
         HIPCHK(c, hipEventRecord(c->ev_a, c->st));
-        for (int q = 0; q < reps; ++q) fused_launch(idx, mode, a, c->n_wg, c->st);
+        for (int q = 0; q < reps; ++q) launch_stage(c, mode, a, &n);
         HIPCHK(c, hipEventRecord(c->ev_b, c->st));
         HIPCHK(c, hipEventSynchronize(c->ev_b));
         HIPCHK(c, hipGetLastError());

@@ -55,12 +55,22 @@ struct FusedArgs {
 struct TileShape { int tx, ty, tz, waves_per_eu; };  // waves_per_eu: occupancy hint given to the compiler
 int fused_shape_count(int scheme);
 TileShape fused_shape(int scheme, int index);
-// Launches the fused kernel of table entry `index`; mode 0 = RK update in
-// one kernel, mode 1 = write dq only, mode 2 = RK update split into an
-// inviscid kernel and a viscous+update kernel.  Returns the dynamic LDS bytes
-// used, or -1.
+// Launches the tile kernels of table entry `index`; mode 0 = RK update,
+// mode 1 = write dq only, mode 2 = RK update with the inviscid part of a
+// characteristic scheme in a kernel of its own.  The component-wise schemes'
+// inviscid dq is in place already (sweep_launch).  Returns the dynamic LDS
+// bytes used, or -1.
 int fused_launch(int index, int mode, const FusedArgs& a, int n_wg, hipStream_t st);
 int fused_lds_bytes(int scheme, int index);
+// Work list of the inviscid sweeps (ostc_kernels_sweep.hip).  x: one workgroup
+// per item, padded points `first` on of the block's interior rows; y, z: one
+// wave per item, 64 columns from `first`, cells c0 .. c0 + n - 1 of each.
+struct SweepItem { int block, first, c0, n; };
+struct SweepPlan { const SweepItem* items[4]; int n[4]; };
+bool sweep_scheme(int scheme);    // component-wise WENO: 50, 51, 71
+int sweep_valid(int scheme);      // padded points a wave of the x sweep advances by
+int visc_cells_per_wg();          // ... and a workgroup of the viscous kernel
+void sweep_launch(const FusedArgs& a, const SweepPlan& s, bool update, hipStream_t st, long long* n);
 void dt_rows(const FusedArgs& a, int n_blocks, int n_wg, double* dt_bits, hipStream_t st, long long* n);
 
 // reverse mode, ostc_kernels_adjoint.hip

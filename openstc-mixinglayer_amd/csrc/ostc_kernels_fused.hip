@@ -1,21 +1,24 @@
-// ostc_kernels_fused.hip -- one persistent kernel per RK stage over the tiles
-// of every block: inviscid WENO fluxes along x, y, z and second-order viscous
-// fluxes staged through LDS, the residual dq kept in registers, and the
-// SSP-RK3 update, primitives and Sutherland viscosity written out (with the
-// sponge layer's relaxation term first where a block has one).  Reads
-// ring slot `in` (state incl. ghosts) and qn = slot 0, writes the interior of
-// slot `out`; ghost layers are filled afterwards by the op launches.
+// ostc_kernels_fused.hip -- the tile kernels of a batched RK stage over the
+// tiles of every block.  k_visc_update: second-order viscous fluxes staged
+// through LDS, added to the stored inviscid residual (ostc_kernels_sweep.hip
+// for the component-wise WENO schemes), then the SSP-RK3 update, primitives
+// and Sutherland viscosity.  k_fused: the characteristic WENO schemes (52,
+// 72) in one launch, their inviscid fluxes along x, y, z staged through LDS
+// and dq kept in registers (with the sponge layer's relaxation term first
+// where a block has one).  Both read ring slot `in` (state incl. ghosts) and
+// qn = slot 0 and write the interior of slot `out`; ghost layers are filled
+// afterwards by the op launches.
 //
 // Work decomposition: a tile is TX x TY x TZ cells of one block, one thread
-// per cell in the cell phases.  Each inviscid direction phase computes split
-// fluxes F+/F- for the tile's (T_d + 2R) x (columns) points, then the WENO
-// flux of every (variable, face) item, then each cell subtracts its face
-// difference.  The viscous phase computes the faces of all three directions
-// as one work list.  Items rather than faces or cells are dealt to the
-// threads, so no wave runs a tail round alone while the others wait at the
-// next barrier.  Accumulation order follows the reference:
+// per cell in the cell phases.  Each inviscid direction phase of k_fused
+// computes split fluxes F+/F- for the tile's (T_d + 2R) x (columns) points,
+// then the WENO flux of every (field, face) item, then each cell subtracts its
+// face difference.  The viscous phase computes the faces of all three
+// directions as one work list.  Items rather than faces or cells are dealt to
+// the threads, so no wave runs a tail round alone while the others wait at
+// the next barrier.  Accumulation order follows the reference:
 // dq = ((0 - dFx) - dFy) - dFz, then + dGx + dGy + dGz (src/RK.cuh:113-139).
-#include "ostc_kernels.hpp"
+#include "ostc_stage.hpp"
 
 namespace ostc {
 
@@ -43,51 +46,39 @@ struct Dir {
   }
 };
 
-// LDS words of one workgroup.  Inviscid phase of direction d: F+ and F- of
-// the 5 variables at the (T_d + 2R) x columns points, plus the WENO epsilon
-// of every face.  Viscous phase: u, v, w, T, mu on the tile box (radius 1)
-// and the 4 viscous fluxes of the faces of all three directions.
-//
-// Two layouts of the inviscid phase.  Compact: the face fluxes overwrite the
-// split fluxes after a barrier, so each thread keeps its items' results in
-// registers until then.  Separate (SEP): the face fluxes and the three
-// per-class epsilons of every face have their own words, so each item writes
-// its result straight to LDS.  And two of the viscous phase: one work list
-// for the faces of all three directions, or (VSPLIT) the x and y faces, then
-// the z faces, with flux words for the larger pass only.  Each choice takes
-// the smaller layout only when the larger one would hold fewer workgroups on
-// a CU than the register budget WPE (waves per SIMD) allows.
-template <int TX, int TY, int TZ, int SCHEME, int WPE>
-struct FusedLds {
+// LDS words of one workgroup.  Characteristic inviscid phase of direction d:
+// F+ and F- of the 5 variables at the (T_d + 2R) x columns points, the face
+// states (AirFace: 9 words, and the WENO epsilon) and the 5 characteristic
+// fluxes of every face.  Viscous phase: u, v, w, T, mu on the tile box
+// (radius 1) and the 4 viscous fluxes of the faces of all three directions:
+// one work list, or (VSPLIT) the x and y faces, then the z faces, with flux
+// words for the larger pass only, where the one list would hold fewer
+// workgroups on a CU than the register budget WPE (waves per SIMD) allows.
+template <int TX, int TY, int TZ, int WPE>
+struct ViscLds {
   static constexpr int NT = TX * TY * TZ;
-  static constexpr int R = Stencil<SCHEME>::R;
-  static constexpr int pts(int td) { return (td + 2 * R) * (NT / td); }
   static constexpr int nf(int td) { return (td + 1) * (NT / td); }
-  static constexpr int mx3(int a, int b, int c) { return a > b ? (a > c ? a : c) : (b > c ? b : c); }
   static constexpr int mx2(int a, int b) { return a > b ? a : b; }
   static constexpr int mn2(int a, int b) { return a < b ? a : b; }
   static constexpr int CU_BYTES = 160 * 1024;
   static constexpr int WGS = mx2(1, WPE * 4 * 64 / NT);  // workgroups per CU the registers allow
   static constexpr int wgs(int words) { return mn2(WGS, CU_BYTES / (words * 8)); }
-  static constexpr int IWORDS = mx3(10 * pts(TX) + nf(TX), 10 * pts(TY) + nf(TY), 10 * pts(TZ) + nf(TZ));
-  static constexpr int IWORDS_SEP =
-      mx3(10 * pts(TX) + 8 * nf(TX), 10 * pts(TY) + 8 * nf(TY), 10 * pts(TZ) + 8 * nf(TZ));
   static constexpr int NB = (TX + 2) * (TY + 2) * (TZ + 2);
-  static constexpr int NFV = nf(TX) + nf(TY) + nf(TZ);
-  static constexpr int VWORDS_ONE = 5 * NB + 4 * NFV;
-  static constexpr int VWORDS_TWO = 5 * NB + 4 * mx2(nf(TX) + nf(TY), nf(TZ));
-  static constexpr bool VSPLIT = wgs(mx2(IWORDS, VWORDS_TWO)) > wgs(mx2(IWORDS, VWORDS_ONE));
-  static constexpr int VWORDS = VSPLIT ? VWORDS_TWO : VWORDS_ONE;
-  static constexpr bool SEP = wgs(mx2(IWORDS_SEP, VWORDS)) >= wgs(mx2(IWORDS, VWORDS));
-  // characteristic schemes (52, 72): split fluxes, the face states (AirFace:
-  // 9 words, and the WENO epsilon) and the 5 characteristic face fluxes
-  static constexpr bool CH = SCHEME == 52 || SCHEME == 72;
-  static constexpr int CH_STATE = 10;
-  static constexpr int IWORDS_CH = mx3(10 * pts(TX) + (CH_STATE + 5) * nf(TX), 10 * pts(TY) + (CH_STATE + 5) * nf(TY),
-                                       10 * pts(TZ) + (CH_STATE + 5) * nf(TZ));
-  static constexpr int WORDS = mx2(CH ? IWORDS_CH : (SEP ? IWORDS_SEP : IWORDS), VWORDS);
+  static constexpr int WORDS_ONE = 5 * NB + 4 * (nf(TX) + nf(TY) + nf(TZ));
+  static constexpr int WORDS_TWO = 5 * NB + 4 * mx2(nf(TX) + nf(TY), nf(TZ));
+  static constexpr bool VSPLIT = wgs(WORDS_TWO) > wgs(WORDS_ONE);
+  static constexpr int WORDS = VSPLIT ? WORDS_TWO : WORDS_ONE;
   static constexpr int BYTES = WORDS * 8;
-  static constexpr int VBYTES = VWORDS * 8;
+};
+
+template <int TX, int TY, int TZ, int SCHEME, int WPE>
+struct FusedLds {
+  using V = ViscLds<TX, TY, TZ, WPE>;
+  static constexpr int R = Stencil<SCHEME>::R;
+  static constexpr int CH_STATE = 10;
+  static constexpr int words(int td) { return 10 * (td + 2 * R) * (V::NT / td) + (CH_STATE + 5) * V::nf(td); }
+  static constexpr int WORDS = V::mx2(V::mx2(words(TX), words(TY)), V::mx2(words(TZ), V::WORDS));
+  static constexpr int BYTES = WORDS * 8;
 };
 
 struct TileCtx {
@@ -95,49 +86,6 @@ struct TileCtx {
   int ti, tj, tk;      // this thread's cell in the tile
   bool valid;          // cell inside the block
 };
-
-template <class T>
-using gptr = __attribute__((address_space(1))) T*;
-
-// What one stage reads and writes of a block, with the arrays as pointers
-// into global memory.  The block table is itself read from memory, so the
-// pointers it holds are generic to the compiler, which would then access
-// every array with flat instructions: those wait on the LDS counter as well
-// and need 64-bit addresses per lane.
-struct StageBlock {
-  int mx, my, mz, g, sx, sy, sz;  // sz fits 32 bits: the host refuses 9 sz >= 2^31
-  int ntx, nty, tile_base, sp_jac;
-  long long n0;
-  gptr<const double> cvi, bvi, muli, qn, jac, met, sp_sigma, sp_mean;
-  gptr<double> cvo, bvo, mulo, mach, dq;
-};
-
-__device__ __forceinline__ StageBlock stage_block(const DevBlock& B, int in, int out) {
-  StageBlock S;
-  S.mx = B.mx; S.my = B.my; S.mz = B.mz; S.g = B.g; S.sx = B.sx; S.sy = B.sy; S.sz = (int)B.sz;
-  S.ntx = B.ntx; S.nty = B.nty; S.tile_base = B.tile_base; S.sp_jac = B.sp_jac;
-  S.n0 = B.n0;
-  S.cvi = (gptr<const double>)B.cv[in];
-  S.bvi = (gptr<const double>)B.bv[in];
-  S.muli = (gptr<const double>)B.mul[in];
-  S.qn = (gptr<const double>)B.cv[0];
-  S.jac = (gptr<const double>)B.jac;
-  S.met = (gptr<const double>)B.met;
-  S.sp_sigma = (gptr<const double>)B.sp_sigma;
-  S.sp_mean = (gptr<const double>)B.sp_mean;
-  S.cvo = (gptr<double>)B.cv[out];
-  S.bvo = (gptr<double>)B.bv[out];
-  S.mulo = (gptr<double>)B.mul[out];
-  S.mach = (gptr<double>)B.mach;
-  S.dq = (gptr<double>)B.dq;
-  return S;
-}
-
-// 32-bit offset of node (i, j, k) in a padded plane; the host refuses blocks
-// whose 9 metric planes would not fit 2^31 doubles.
-__device__ __forceinline__ int poff(const StageBlock& b, int i, int j, int k) {
-  return ((k + b.g) * b.sy + (j + b.g)) * b.sx + (i + b.g);
-}
 
 // The block coordinates of face f of direction D (its lower node L along D,
 // face L+1/2) and whether the face lies in the block (faces past the end of a
@@ -286,16 +234,14 @@ __device__ __forceinline__ void characteristic_faces(double* smem, const StageBl
 }
 
 // Inviscid fluxes along direction D, subtracted from dq.  The face work is
-// spread over (variable, face) items, 5 NF of them for NT threads, so every
+// spread over (field, face) items, 5 NF of them for NT threads, so every
 // wave carries the same share whatever NF mod NT is.
-template <int TX, int TY, int TZ, int SCHEME, int WPE, int D>
+template <int TX, int TY, int TZ, int SCHEME, int D>
 __device__ __forceinline__ void inviscid_phase(double* smem, const StageBlock& B, const Params& P,
                                                const TileCtx& t, double dq[5]) {
   using Dr = Dir<TX, TY, TZ, D>;
-  constexpr int NT = Dr::NT, R = Stencil<SCHEME>::R, W = Stencil<SCHEME>::W;
-  constexpr int TD = Dr::TD, PC = Dr::PC, LP = TD + 2 * R, NPTS = LP * PC, NF = Dr::NF;
-  constexpr int NI = 5 * NF, IPT = (NI + NT - 1) / NT;
-  constexpr bool SEP = FusedLds<TX, TY, TZ, SCHEME, WPE>::SEP;
+  constexpr int NT = Dr::NT, R = Stencil<SCHEME>::R;
+  constexpr int PC = Dr::PC, LP = Dr::TD + 2 * R, NPTS = LP * PC;
   const int tid = threadIdx.x;
   const int origin = D == 0 ? t.i0 : (D == 1 ? t.j0 : t.k0);
   const gptr<const double> cv = B.cvi;
@@ -303,7 +249,6 @@ __device__ __forceinline__ void inviscid_phase(double* smem, const StageBlock& B
   const int s = B.sz;
   double* sFp = smem;
   double* sFm = smem + 5 * NPTS;
-  double* sEps = smem + 10 * NPTS;  // SEP: [3][NF], the epsilon of rho, of the momenta and of the energy
 
   // split fluxes at the points of every column
   for (int p = tid; p < NPTS; p += NT) {
@@ -331,114 +276,7 @@ __device__ __forceinline__ void inviscid_phase(double* smem, const StageBlock& B
       for (int l = 0; l < 5; ++l) { sFp[l * NPTS + p] = fp[l]; sFm[l * NPTS + p] = fm[l]; }
     }
   }
-  if constexpr (Stencil<SCHEME>::CH) {
-    characteristic_faces<TX, TY, TZ, SCHEME, D>(smem, B, P, t, dq);
-    return;
-  }
-  // the epsilon of every face (src/WENO.cu:1469-1482), shared by its 5 items
-  for (int f = tid; f < NF; f += NT) {
-    int ijk[3];
-    if (face_node<TX, TY, TZ, D>(B, t, f, ijk)) {
-      const int p1 = poff(B, ijk[0], ijk[1], ijk[2]);
-      const int p2 = p1 + (D == 0 ? 1 : (D == 1 ? B.sx : B.sx * B.sy));
-      const double j1 = B.jac[p1], j2 = B.jac[p2];
-      double eps3[3];
-      weno_eps(P, B.met[p1 + 3 * D * s] * j1, B.met[p1 + (3 * D + 1) * s] * j1, B.met[p1 + (3 * D + 2) * s] * j1,
-               B.met[p2 + 3 * D * s] * j2, B.met[p2 + (3 * D + 1) * s] * j2, B.met[p2 + (3 * D + 2) * s] * j2,
-               eps3);
-      sEps[f] = eps3[0];
-      if (SEP) {
-        sEps[NF + f] = eps3[1];
-        sEps[2 * NF + f] = eps3[2];
-      }
-    }
-  }
-  __syncthreads();
-
-  if constexpr (SEP) {
-    double* sFc = smem + 10 * NPTS + 3 * NF;  // [5][NF]
-#pragma unroll 1
-    for (int it = tid; it < NI; it += NT) {
-      const int l = it / NF, f = it - l * NF;
-      double val = 0.0;
-      int ijk[3];
-      if (face_node<TX, TY, TZ, D>(B, t, f, ijk)) {
-        int col, sf;
-        Dr::face(f, col, sf);
-        const int sL = sf - 1 + R;
-        const double e = sEps[(l == 0 ? 0 : (l == 4 ? 2 : 1)) * NF + f];
-        const double* fpl = sFp + l * NPTS;
-        const double* fml = sFm + l * NPTS;
-        double vp[W], vm[W];
-#pragma unroll
-        for (int r = 0; r < W; ++r) {
-          vp[r] = fpl[Dr::template at<LP>(col, sL - W / 2 + r)];
-          vm[r] = fml[Dr::template at<LP>(col, sL - W / 2 + 1 + r)];
-        }
-        val = weno_face<SCHEME>(vp, vm, e);
-      }
-      sFc[it] = val;
-    }
-    __syncthreads();
-    if (t.valid) {
-      const int col = Dr::my_col(t.ti, t.tj, t.tk), pos = Dr::my_pos(t.ti, t.tj, t.tk);
-      const int fL = Dr::template at<TD + 1>(col, pos), fR = Dr::template at<TD + 1>(col, pos + 1);
-#pragma unroll
-      for (int l = 0; l < 5; ++l) dq[l] -= sFc[l * NF + fR] - sFc[l * NF + fL];
-    }
-    __syncthreads();
-    return;
-  }
-
-  // one item per iteration (the loop is not unrolled, so the WENO evaluations
-  // of different items do not overlap in registers); each result is kept in
-  // its own register through a chain of selects
-  double fres[IPT];
-#pragma unroll
-  for (int u = 0; u < IPT; ++u) fres[u] = 0.0;
-#pragma unroll 1
-  for (int u = 0; u < IPT; ++u) {
-    const int it = tid + u * NT;
-    double val = 0.0;
-    if (it < NI) {
-      const int l = it / NF, f = it - l * NF;
-      int ijk[3];
-      if (face_node<TX, TY, TZ, D>(B, t, f, ijk)) {
-        int col, sf;
-        Dr::face(f, col, sf);
-        const int sL = sf - 1 + R;
-        // eps_scaled of src/WENO.cu:1478-1481 for variable l
-        const double e0 = sEps[f];
-        const double e = l == 0 ? e0 : (l == 4 ? e0 * P.v_ref * P.v_ref * P.v_ref * P.v_ref : e0 * P.v_ref * P.v_ref);
-        const double* fpl = sFp + l * NPTS;
-        const double* fml = sFm + l * NPTS;
-        double vp[W], vm[W];
-#pragma unroll
-        for (int r = 0; r < W; ++r) {
-          vp[r] = fpl[Dr::template at<LP>(col, sL - W / 2 + r)];
-          vm[r] = fml[Dr::template at<LP>(col, sL - W / 2 + 1 + r)];
-        }
-        val = weno_face<SCHEME>(vp, vm, e);
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < IPT; ++q) fres[q] = q == u ? val : fres[q];
-  }
-  __syncthreads();
-  double* sFc = smem;  // [5][NF], aliases the split fluxes, which are no longer read
-#pragma unroll
-  for (int u = 0; u < IPT; ++u) {
-    const int it = tid + u * NT;
-    if (it < NI) sFc[it] = fres[u];
-  }
-  __syncthreads();
-  if (t.valid) {
-    const int col = Dr::my_col(t.ti, t.tj, t.tk), pos = Dr::my_pos(t.ti, t.tj, t.tk);
-    const int fL = Dr::template at<TD + 1>(col, pos), fR = Dr::template at<TD + 1>(col, pos + 1);
-#pragma unroll
-    for (int l = 0; l < 5; ++l) dq[l] -= sFc[l * NF + fR] - sFc[l * NF + fL];
-  }
-  __syncthreads();
+  characteristic_faces<TX, TY, TZ, SCHEME, D>(smem, B, P, t, dq);
 }
 
 // Viscous flux of face f of direction D (src/ViscousScheme.cuh:23-909),
@@ -595,104 +433,136 @@ __device__ __forceinline__ void viscous_phase(double* smem, const StageBlock& B,
   __syncthreads();
 }
 
-// MODE 0: inviscid + viscous + RK update; MODE 1: write dq (inviscid, and
-// viscous when VISC) without updating; MODE 2: viscous + RK update starting
-// from the inviscid dq that a MODE 1 / VISC 0 launch stored (a stage split in
-// two kernels of lower register and LDS pressure).
-template <int TX, int TY, int TZ, int WPE, int SCHEME, int VISC, int MODE>
-__global__ __launch_bounds__(TX * TY * TZ) __attribute__((amdgpu_waves_per_eu(WPE))) void k_fused(FusedArgs A) {
-  constexpr int NT = TX * TY * TZ;
-  extern __shared__ double smem[];
-  const int tid = threadIdx.x;
-  TileCtx t;
-  t.ti = tid % TX;
-  t.tj = (tid / TX) % TY;
-  t.tk = tid / (TX * TY);
-  // tile assignment.  Round-robin dispatch puts workgroup w on XCD w % 8;
-  // with xcd_remap the workgroups of one XCD take consecutive work items
-  // (XCD x owns items [x q + min(x, r), ...) of G = 8 q + r), so tiles that
-  // run together on one XCD are neighbours in the block and share their
-  // halo points through that XCD's L2.  One workgroup per tile: item = tile;
-  // a persistent grid: item = a chunk of consecutive tiles.
+// The tiles of workgroup blockIdx.x: first, first + step, ... < last.
+// Round-robin dispatch puts workgroup w on XCD w % 8; with xcd_remap the
+// workgroups of one XCD take consecutive work items (XCD x owns items
+// [x q + min(x, r), ...) of G = 8 q + r), so tiles that run together on one
+// XCD are neighbours in the block and share their halo points through that
+// XCD's L2.  One workgroup per tile: item = tile; a persistent grid: item = a
+// chunk of consecutive tiles.
+struct TileRange { int first, last, step; };
+__device__ __forceinline__ TileRange tile_range(const FusedArgs& A) {
   const int G = gridDim.x;
   int lid = blockIdx.x;
   if (A.xcd_remap) {
     const int x = blockIdx.x % 8, q = G / 8, r = G % 8;
     lid = x * q + min(x, r) + blockIdx.x / 8;
   }
-  int first, step, last;
   if (G < A.n_tiles && A.xcd_remap) {
     const int chunk = (A.n_tiles + G - 1) / G;
-    first = lid * chunk;
-    last = min(A.n_tiles, first + chunk);
-    step = 1;
-  } else {
-    first = lid;
-    last = A.n_tiles;
-    step = G;
+    return TileRange{lid * chunk, min(A.n_tiles, (lid + 1) * chunk), 1};
   }
-  for (int tile = first; tile < last; tile += step) {
+  return TileRange{lid, A.n_tiles, G};
+}
+
+// The block of `tile` (its descriptor is read from memory once per tile into
+// the stage's view) and this thread's cell in it.
+template <int TX, int TY, int TZ>
+__device__ __forceinline__ StageBlock tile_block(const FusedArgs& A, int tile, int b, TileCtx& t) {
+  const StageBlock B = stage_block(A.blocks[b], A.in, A.out);
+  const int tid = threadIdx.x;
+  t.ti = tid % TX;
+  t.tj = (tid / TX) % TY;
+  t.tk = tid / (TX * TY);
+  const int local = tile - B.tile_base;
+  t.i0 = (local % B.ntx) * TX;
+  t.j0 = ((local / B.ntx) % B.nty) * TY;
+  t.k0 = (local / (B.ntx * B.nty)) * TZ;
+  t.valid = t.i0 + t.ti < B.mx && t.j0 + t.tj < B.my && t.k0 + t.tk < B.mz;
+  return B;
+}
+
+// update_cv_and_bv_rk<Air> (src/RK.cuh:230-284) and the interior part of
+// update_physical_properties<Air> (src/FieldOperation.cuh:107-140) of cell (i, j, k).
+__device__ __forceinline__ void stage_update(const FusedArgs& A, const StageBlock& B, int i, int j, int k,
+                                             const double dq[5]) {
+  const int p = poff(B, i, j, k), s = B.sz;
+  const double dt = *A.dt;
+  const double dt_div_jac = dt / B.jac[p];
+  double c[5];
+#pragma unroll
+  for (int l = 0; l < 5; ++l) {
+    c[l] = A.ra * B.qn[p + l * s] + A.rb * B.cvi[p + l * s] + A.rc * dt_div_jac * dq[l];
+    B.cvo[p + l * s] = c[l];
+  }
+  const double density_inv = 1.0 / c[0];
+  const double u = c[1] * density_inv, v = c[2] * density_inv, w = c[3] * density_inv;
+  const double V2 = u * u + v * v + w * w;
+  const double pr = (kGamma - 1) * (c[4] - 0.5 * c[0] * V2);
+  const double T = pr * kMwAir * density_inv / kRu;
+  B.bvo[p] = c[0];
+  B.bvo[p + s] = u;
+  B.bvo[p + 2 * s] = v;
+  B.bvo[p + 3 * s] = w;
+  B.bvo[p + 4 * s] = pr;
+  B.bvo[p + 5 * s] = T;
+  constexpr double c_temp{kGamma * kRu / kMwAir};
+  B.mulo[p] = sutherland(T);
+  B.mach[p] = sqrt(V2) / sqrt(c_temp * T);
+}
+
+// Viscous fluxes (VISC) and the RK update, starting from the stored inviscid
+// dq; UPDATE false: the viscous fluxes are added to the stored dq instead.
+template <int TX, int TY, int TZ, int WPE, int VISC, bool UPDATE>
+__global__ __launch_bounds__(TX * TY * TZ) __attribute__((amdgpu_waves_per_eu(WPE))) void k_visc_update(FusedArgs A) {
+  extern __shared__ double smem[];
+  TileCtx t;
+  const TileRange r = tile_range(A);
+  for (int tile = r.first; tile < r.last; tile += r.step) {
     const int b = A.tile_block[tile];
     if (A.target_block >= 0 && b != A.target_block) continue;
-    // the descriptor is read from memory once per tile into the stage's view
-    const StageBlock B = stage_block(A.blocks[b], A.in, A.out);
-    const int local = tile - B.tile_base;
-    t.i0 = (local % B.ntx) * TX;
-    t.j0 = ((local / B.ntx) % B.nty) * TY;
-    t.k0 = (local / (B.ntx * B.nty)) * TZ;
+    const StageBlock B = tile_block<TX, TY, TZ>(A, tile, b, t);
     const int i = t.i0 + t.ti, j = t.j0 + t.tj, k = t.k0 + t.tk;
-    t.valid = i < B.mx && j < B.my && k < B.mz;
-    const long long q0 = ((long long)k * B.my + j) * B.mx + i;  // interior index (dq, sponge planes)
+    const int q0 = (k * B.my + j) * B.mx + i, n0 = (int)B.n0;
     double dq[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    if (MODE != 2 && B.sp_sigma && t.valid) {
+    if (t.valid) {
+#pragma unroll
+      for (int l = 0; l < 5; ++l) dq[l] = B.dq[q0 + l * n0];
+    }
+    if (VISC) viscous_phase<TX, TY, TZ, ViscLds<TX, TY, TZ, WPE>::VSPLIT>(smem, B, A.P, t, dq);
+    if (!t.valid) continue;
+    if constexpr (UPDATE) {
+      stage_update(A, B, i, j, k, dq);
+    } else {
+#pragma unroll
+      for (int l = 0; l < 5; ++l) B.dq[q0 + l * n0] = dq[l];
+    }
+  }
+}
+
+// Characteristic schemes.  UPDATE true: inviscid + viscous (VISC) + RK
+// update; false: the residual is written to dq.
+template <int TX, int TY, int TZ, int WPE, int SCHEME, int VISC, bool UPDATE>
+__global__ __launch_bounds__(TX * TY * TZ) __attribute__((amdgpu_waves_per_eu(WPE))) void k_fused(FusedArgs A) {
+  extern __shared__ double smem[];
+  TileCtx t;
+  const TileRange r = tile_range(A);
+  for (int tile = r.first; tile < r.last; tile += r.step) {
+    const int b = A.tile_block[tile];
+    if (A.target_block >= 0 && b != A.target_block) continue;
+    const StageBlock B = tile_block<TX, TY, TZ>(A, tile, b, t);
+    const int i = t.i0 + t.ti, j = t.j0 + t.tj, k = t.k0 + t.tk;
+    const int q0 = (k * B.my + j) * B.mx + i, n0 = (int)B.n0;  // interior index (dq, sponge planes)
+    double dq[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    if (B.sp_sigma && t.valid) {
       // sponge_layer_source (src/SpongeLayer.cu:68-160), the first term of the
       // stage's dq as in compute_source: dq -= sigma (cv - mean)
       const int p = poff(B, i, j, k), s = B.sz;
       const double sigma = B.sp_jac ? B.sp_sigma[q0] * B.jac[p] : B.sp_sigma[q0];
 #pragma unroll
-      for (int l = 0; l < 5; ++l) dq[l] -= sigma * (B.cvi[p + l * s] - B.sp_mean[q0 + l * B.n0]);
+      for (int l = 0; l < 5; ++l) dq[l] -= sigma * (B.cvi[p + l * s] - B.sp_mean[q0 + l * n0]);
     }
-    if (MODE != 2) {
-      inviscid_phase<TX, TY, TZ, SCHEME, WPE, 0>(smem, B, A.P, t, dq);
-      inviscid_phase<TX, TY, TZ, SCHEME, WPE, 1>(smem, B, A.P, t, dq);
-      inviscid_phase<TX, TY, TZ, SCHEME, WPE, 2>(smem, B, A.P, t, dq);
-    } else if (t.valid) {
-      // split stage: the inviscid part of dq was written by the MODE 1 launch
-#pragma unroll
-      for (int l = 0; l < 5; ++l) dq[l] = B.dq[q0 + l * B.n0];
-    }
-    if (VISC) viscous_phase<TX, TY, TZ, FusedLds<TX, TY, TZ, SCHEME, WPE>::VSPLIT>(smem, B, A.P, t, dq);
+    inviscid_phase<TX, TY, TZ, SCHEME, 0>(smem, B, A.P, t, dq);
+    inviscid_phase<TX, TY, TZ, SCHEME, 1>(smem, B, A.P, t, dq);
+    inviscid_phase<TX, TY, TZ, SCHEME, 2>(smem, B, A.P, t, dq);
+    if (VISC) viscous_phase<TX, TY, TZ, ViscLds<TX, TY, TZ, WPE>::VSPLIT>(smem, B, A.P, t, dq);
     if (!t.valid) continue;
-    const int p = poff(B, i, j, k), s = B.sz;
-    if (MODE == 1) {
+    if constexpr (UPDATE) {
+      stage_update(A, B, i, j, k, dq);
+    } else {
 #pragma unroll
-      for (int l = 0; l < 5; ++l) B.dq[q0 + l * B.n0] = dq[l];
-      continue;
+      for (int l = 0; l < 5; ++l) B.dq[q0 + l * n0] = dq[l];
     }
-    // update_cv_and_bv_rk<Air> (src/RK.cuh:230-284) and the interior part of
-    // update_physical_properties<Air> (src/FieldOperation.cuh:107-140)
-    const double dt = *A.dt;
-    const double dt_div_jac = dt / B.jac[p];
-    double c[5];
-#pragma unroll
-    for (int l = 0; l < 5; ++l) {
-      c[l] = A.ra * B.qn[p + l * s] + A.rb * B.cvi[p + l * s] + A.rc * dt_div_jac * dq[l];
-      B.cvo[p + l * s] = c[l];
-    }
-    const double density_inv = 1.0 / c[0];
-    const double u = c[1] * density_inv, v = c[2] * density_inv, w = c[3] * density_inv;
-    const double V2 = u * u + v * v + w * w;
-    const double pr = (kGamma - 1) * (c[4] - 0.5 * c[0] * V2);
-    const double T = pr * kMwAir * density_inv / kRu;
-    B.bvo[p] = c[0];
-    B.bvo[p + s] = u;
-    B.bvo[p + 2 * s] = v;
-    B.bvo[p + 3 * s] = w;
-    B.bvo[p + 4 * s] = pr;
-    B.bvo[p + 5 * s] = T;
-    constexpr double c_temp{kGamma * kRu / kMwAir};
-    B.mulo[p] = sutherland(T);
-    B.mach[p] = sqrt(V2) / sqrt(c_temp * T);
   }
 }
 
@@ -766,47 +636,64 @@ static constexpr int kNumShapes = sizeof(kShapes) / sizeof(kShapes[0]);
 int fused_shape_count(int) { return kNumShapes; }
 TileShape fused_shape(int, int index) { return kShapes[index]; }
 
-template <int TX, int TY, int TZ, int WPE, int SCHEME>
-static int launch_shape(int mode, int visc, const FusedArgs& a, int n_wg, hipStream_t st) {
-  constexpr int bytes = FusedLds<TX, TY, TZ, SCHEME, WPE>::BYTES;
-  constexpr int vbytes = FusedLds<TX, TY, TZ, SCHEME, WPE>::VBYTES;
-  if (bytes > 160 * 1024) return -1;
-  static bool attr_set = false;  // dynamic LDS above 64 KiB has to be enabled per kernel
-  if (!attr_set) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_fused<TX, TY, TZ, WPE, SCHEME, 1, 2>),
-                        hipFuncAttributeMaxDynamicSharedMemorySize, vbytes);
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_fused<TX, TY, TZ, WPE, SCHEME, 1, 0>),
-                        hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_fused<TX, TY, TZ, WPE, SCHEME, 0, 0>),
-                        hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_fused<TX, TY, TZ, WPE, SCHEME, 1, 1>),
-                        hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_fused<TX, TY, TZ, WPE, SCHEME, 0, 1>),
-                        hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+// Dynamic LDS above 64 KiB has to be enabled per kernel, once.
+template <class K>
+static void allow_lds(K kernel, int bytes) {
+  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+}
+
+template <int TX, int TY, int TZ, int WPE>
+static void launch_visc(bool update, const FusedArgs& a, int n_wg, hipStream_t st) {
+  constexpr int bytes = ViscLds<TX, TY, TZ, WPE>::BYTES;
+  static bool attr_set = false;
+  if (bytes > 64 * 1024 && !attr_set) {
+    allow_lds(&k_visc_update<TX, TY, TZ, WPE, 1, true>, bytes);
+    allow_lds(&k_visc_update<TX, TY, TZ, WPE, 1, false>, bytes);
     attr_set = true;
   }
   const dim3 grid(n_wg), block(TX * TY * TZ);
-  if (mode == 2 && visc) {  // split stage
-    hipLaunchKernelGGL((k_fused<TX, TY, TZ, WPE, SCHEME, 0, 1>), grid, block, bytes, st, a);
-    hipLaunchKernelGGL((k_fused<TX, TY, TZ, WPE, SCHEME, 1, 2>), grid, block, vbytes, st, a);
+  if (!a.P.visc) {
+    if (update) hipLaunchKernelGGL((k_visc_update<TX, TY, TZ, WPE, 0, true>), grid, block, 0, st, a);
+    return;
+  }
+  if (update) hipLaunchKernelGGL((k_visc_update<TX, TY, TZ, WPE, 1, true>), grid, block, bytes, st, a);
+  else hipLaunchKernelGGL((k_visc_update<TX, TY, TZ, WPE, 1, false>), grid, block, bytes, st, a);
+}
+
+template <int TX, int TY, int TZ, int WPE, int SCHEME>
+static int launch_shape(int mode, const FusedArgs& a, int n_wg, hipStream_t st) {
+  constexpr int bytes = FusedLds<TX, TY, TZ, SCHEME, WPE>::BYTES;
+  if (bytes > 160 * 1024) return -1;
+  static bool attr_set = false;
+  if (!attr_set) {
+    allow_lds(&k_fused<TX, TY, TZ, WPE, SCHEME, 1, true>, bytes);
+    allow_lds(&k_fused<TX, TY, TZ, WPE, SCHEME, 0, true>, bytes);
+    allow_lds(&k_fused<TX, TY, TZ, WPE, SCHEME, 1, false>, bytes);
+    allow_lds(&k_fused<TX, TY, TZ, WPE, SCHEME, 0, false>, bytes);
+    attr_set = true;
+  }
+  const dim3 grid(n_wg), block(TX * TY * TZ);
+  if (mode == 2 && a.P.visc) {  // split stage
+    hipLaunchKernelGGL((k_fused<TX, TY, TZ, WPE, SCHEME, 0, false>), grid, block, bytes, st, a);
+    launch_visc<TX, TY, TZ, WPE>(true, a, n_wg, st);
     return bytes;
   }
   if (mode == 2) mode = 0;
-  if (mode == 0 && visc) hipLaunchKernelGGL((k_fused<TX, TY, TZ, WPE, SCHEME, 1, 0>), grid, block, bytes, st, a);
-  else if (mode == 0) hipLaunchKernelGGL((k_fused<TX, TY, TZ, WPE, SCHEME, 0, 0>), grid, block, bytes, st, a);
-  else if (visc) hipLaunchKernelGGL((k_fused<TX, TY, TZ, WPE, SCHEME, 1, 1>), grid, block, bytes, st, a);
-  else hipLaunchKernelGGL((k_fused<TX, TY, TZ, WPE, SCHEME, 0, 1>), grid, block, bytes, st, a);
+  if (mode == 0 && a.P.visc) hipLaunchKernelGGL((k_fused<TX, TY, TZ, WPE, SCHEME, 1, true>), grid, block, bytes, st, a);
+  else if (mode == 0) hipLaunchKernelGGL((k_fused<TX, TY, TZ, WPE, SCHEME, 0, true>), grid, block, bytes, st, a);
+  else if (a.P.visc) hipLaunchKernelGGL((k_fused<TX, TY, TZ, WPE, SCHEME, 1, false>), grid, block, bytes, st, a);
+  else hipLaunchKernelGGL((k_fused<TX, TY, TZ, WPE, SCHEME, 0, false>), grid, block, bytes, st, a);
   return bytes;
 }
 
 template <int TX, int TY, int TZ, int WPE>
 static int launch_scheme(int mode, const FusedArgs& a, int n_wg, hipStream_t st) {
   switch (a.P.scheme) {
-    case 51: return launch_shape<TX, TY, TZ, WPE, 51>(mode, a.P.visc, a, n_wg, st);
-    case 50: return launch_shape<TX, TY, TZ, WPE, 50>(mode, a.P.visc, a, n_wg, st);
-    case 71: return launch_shape<TX, TY, TZ, WPE, 71>(mode, a.P.visc, a, n_wg, st);
-    case 52: return launch_shape<TX, TY, TZ, WPE, 52>(mode, a.P.visc, a, n_wg, st);
-    case 72: return launch_shape<TX, TY, TZ, WPE, 72>(mode, a.P.visc, a, n_wg, st);
+    case 50:
+    case 51:
+    case 71: launch_visc<TX, TY, TZ, WPE>(mode != 1, a, n_wg, st); return ViscLds<TX, TY, TZ, WPE>::BYTES;
+    case 52: return launch_shape<TX, TY, TZ, WPE, 52>(mode, a, n_wg, st);
+    case 72: return launch_shape<TX, TY, TZ, WPE, 72>(mode, a, n_wg, st);
     default: return -1;
   }
 }
@@ -825,10 +712,9 @@ int fused_lds_bytes(int scheme, int index) {
   int i = 0;
 #define X(a_, b_, c_, w_)                                                        \
   if (index == i) {                                                          \
-    if (scheme == 71) return FusedLds<a_, b_, c_, 71, w_>::BYTES;            \
     if (scheme == 52) return FusedLds<a_, b_, c_, 52, w_>::BYTES;            \
     if (scheme == 72) return FusedLds<a_, b_, c_, 72, w_>::BYTES;            \
-    return FusedLds<a_, b_, c_, 51, w_>::BYTES;                              \
+    return ViscLds<a_, b_, c_, w_>::BYTES;                                   \
   }                                                                          \
   ++i;
   OSTC_SHAPES(X)
