@@ -79,6 +79,16 @@ struct ostc_fr_ctx_s {
   hipGraph_t graph = nullptr;
   hipGraphExec_t gexec = nullptr;
   long long graph_launches = 0;
+  // Ghost-layer ops and the workgroups that run them.  Boundary faces in
+  // rounds (the r-th face of every block, blocks being independent), inner
+  // faces in levels whose ops touch no common node; a range of workgroups
+  // for every group and for every op.
+  FrBlockDev* d_blocks = nullptr;
+  GhostOp* d_ghost = nullptr;
+  GhostWg* d_ghost_wg = nullptr;
+  struct WgRange { int lo = 0, n = 0; bool far = false; };  // far: holds a farfield face
+  std::vector<WgRange> bc_rounds, comm_levels, plain_comm;  // plain_comm: inner faces in the reference's order
+  std::vector<std::vector<WgRange>> plain_bc;               // per block, in the order of application
   // batched step: the per-block kernel arguments and its own graph
   std::vector<FrArgs> h_args;
   hipGraph_t bgraph = nullptr;
@@ -154,48 +164,159 @@ int bc_priority(int type) {
   return type == OSTC_BC_FARFIELD ? 0 : (type == OSTC_BC_OUTFLOW ? 1 : (type == OSTC_BC_INFLOW ? 2 : 3));
 }
 
-// Boundary conditions of one block (priority order, then registration
-// order), src/BoundCond.cuh:1488-1678.
-void apply_bc(ostc_fr_ctx c, int b, long long* n) {
-  std::vector<FaceDesc> fs = c->blocks[b].faces;
-  std::stable_sort(fs.begin(), fs.end(),
-                   [](const FaceDesc& x, const FaceDesc& y) { return bc_priority(x.type) < bc_priority(y.type); });
-  const FrArgs a = args(c, b);
-  for (const FaceDesc& f : fs) {
-    FaceBox fb{};
-    for (int d = 0; d < 3; ++d) {
-      fb.lo[d] = f.r.lo[d];
-      fb.n[d] = f.r.hi[d] - f.r.lo[d] + 1;
-    }
-    fb.axis = f.r.axis;
-    fb.side = f.r.side;
-    const double* ff = f.type == OSTC_BC_FARFIELD ? c->d_ff + (size_t)f.ff * 26
-                       : f.type == OSTC_BC_INFLOW ? c->d_inflow + (size_t)f.ff * ostc::kInflowDoubles
-                                                  : nullptr;
-    launch_bc(a, c->ns, fb, f.type, ff, f.type == OSTC_BC_INFLOW ? c->d_inflow + f.y_off : nullptr, c->d_pass + b,
-              c->st, n);
-  }
-  if (c->inflow_noise) launch_count_pass(c->d_pass + b, c->st, n);
+void ghost(ostc_fr_ctx c, const ostc_fr_ctx_s::WgRange& w, long long* n) {
+  launch_ghost(c->h_args[0], c->ns, c->d_blocks, c->d_ghost, c->d_ghost_wg + w.lo, w.n, w.far, c->st, n);
 }
 
-// data_communication, inner faces in block order then face order
-// (src/DataCommunication.cuh:29-58).
-void exchange(ostc_fr_ctx c, long long* n) {
-  for (size_t b = 0; b < c->blocks.size(); ++b) {
-    const FrArgs a = args(c, (int)b);
-    for (const FaceMap& f : c->blocks[b].inner) {
-      CommMap m{};
-      for (int d = 0; d < 3; ++d) {
-        m.lo[d] = f.lo[d];
-        m.n[d] = f.hi[d] - f.lo[d] + 1;
-        m.code[d] = f.code[d];
-        m.off[d] = f.off[d];
-      }
-      m.axis = f.axis;
-      m.shared = f.shared;
-      launch_comm(a, c->blocks[f.target].d, c->ns, m, c->st, n);
+struct Box { int lo[3], hi[3]; };  // inclusive
+struct Access { int block; Box box; };
+
+bool meet(const std::vector<Access>& x, const std::vector<Access>& y) {
+  for (auto& u : x)
+    for (auto& v : y) {
+      bool hit = u.block == v.block;
+      for (int d = 0; d < 3; ++d) hit = hit && u.box.lo[d] <= v.box.hi[d] && v.box.lo[d] <= u.box.hi[d];
+      if (hit) return true;
     }
+  return false;
+}
+
+// Builds the ghost-layer ops.  Boundary conditions: priority order, then
+// registration order (src/BoundCond.cuh:1488-1678).  Inner faces: the
+// reference runs them in block order, then face order
+// (src/DataCommunication.cuh:29-58); a face's level is one more than the
+// highest level of an earlier face that writes what it reads or writes, or
+// reads what it writes, so the levels in order give the sequential result.
+int build_ghost(ostc_fr_ctx c) {
+  const int nb = (int)c->blocks.size();
+  std::vector<GhostOp> ops;
+  std::vector<GhostWg> wgs;
+  auto append = [&](int q) {  // the workgroups of op q
+    const GhostOp& o = ops[q];
+    ostc_fr_ctx_s::WgRange r;
+    r.lo = (int)wgs.size();
+    const int items = o.n[0] * o.n[1] * o.n[2] * o.layers;
+    for (int f = 0; f < items; f += kGhostWg) wgs.push_back(GhostWg{q, f});
+    r.n = (int)wgs.size() - r.lo;
+    r.far = o.type == GHOST_FARFIELD;
+    return r;
+  };
+  std::vector<std::vector<int>> faces(nb);
+  size_t rounds = 0;
+  for (int b = 0; b < nb; ++b) {
+    const HBlock& B = c->blocks[b];
+    std::vector<FaceDesc> fs = B.faces;
+    std::stable_sort(fs.begin(), fs.end(),
+                     [](const FaceDesc& x, const FaceDesc& y) { return bc_priority(x.type) < bc_priority(y.type); });
+    for (const FaceDesc& f : fs) {
+      GhostOp o{};
+      o.type = f.type == OSTC_BC_FARFIELD ? GHOST_FARFIELD
+               : f.type == OSTC_BC_INFLOW ? GHOST_INFLOW
+               : f.type == OSTC_BC_PERIODIC ? GHOST_PERIODIC
+                                            : GHOST_OUTFLOW;
+      o.block = b;
+      o.axis = f.r.axis;
+      o.side = f.r.side;
+      for (int d = 0; d < 3; ++d) {
+        o.lo[d] = f.r.lo[d];
+        o.n[d] = f.r.hi[d] - f.r.lo[d] + 1;
+      }
+      o.layers = o.type == GHOST_OUTFLOW || o.type == GHOST_PERIODIC ? c->ngg : 1;
+      if (f.type == OSTC_BC_FARFIELD) o.ff = c->d_ff + (size_t)f.ff * 26;
+      if (f.type == OSTC_BC_INFLOW) {
+        o.ff = c->d_inflow + (size_t)f.ff * ostc::kInflowDoubles;
+        o.y = c->d_inflow + f.y_off;
+      }
+      o.pass = c->d_pass + b;
+      faces[b].push_back((int)ops.size());
+      ops.push_back(o);
+    }
+    rounds = std::max(rounds, faces[b].size());
   }
+  c->plain_bc.assign(nb, {});
+  c->bc_rounds.clear();
+  for (size_t r = 0; r < rounds; ++r) {
+    ostc_fr_ctx_s::WgRange g;
+    g.lo = (int)wgs.size();
+    for (int b = 0; b < nb; ++b)
+      if (r < faces[b].size()) {
+        c->plain_bc[b].push_back(append(faces[b][r]));
+        g.far = g.far || c->plain_bc[b].back().far;
+      }
+    g.n = (int)wgs.size() - g.lo;
+    c->bc_rounds.push_back(g);
+  }
+  struct Inner { int op, level; std::vector<Access> w, r; };
+  std::vector<Inner> inner;
+  int levels = 0;
+  for (int b = 0; b < nb; ++b)
+    for (const FaceMap& f : c->blocks[b].inner) {
+      GhostOp o{};
+      o.type = GHOST_INNER;
+      o.block = b;
+      o.target = f.target;
+      o.axis = f.axis;
+      o.layers = 1;
+      o.shared = f.shared;
+      Box box, sh;
+      for (int d = 0; d < 3; ++d) {
+        o.lo[d] = box.lo[d] = sh.lo[d] = f.lo[d];
+        box.hi[d] = sh.hi[d] = f.hi[d];
+        o.n[d] = f.hi[d] - f.lo[d] + 1;
+        o.code[d] = f.code[d];
+        o.off[d] = f.off[d];
+      }
+      sh.lo[f.axis] = sh.hi[f.axis] = f.shared;
+      auto image = [&](const Box& s) {
+        Box t;
+        for (int d = 0; d < 3; ++d) {
+          const int code = f.code[d], a = (code < 0 ? -code : code) - 1;
+          const int x = f.off[d] + (code < 0 ? -s.lo[a] : s.lo[a]), y = f.off[d] + (code < 0 ? -s.hi[a] : s.hi[a]);
+          t.lo[d] = std::min(x, y);
+          t.hi[d] = std::max(x, y);
+        }
+        return t;
+      };
+      Inner e{(int)ops.size(), 0, {{b, box}, {f.target, image(sh)}}, {{f.target, image(box)}, {b, sh}}};
+      for (const Inner& x : inner)
+        if (meet(x.w, e.w) || meet(x.w, e.r) || meet(x.r, e.w)) e.level = std::max(e.level, x.level + 1);
+      levels = std::max(levels, e.level + 1);
+      inner.push_back(e);
+      ops.push_back(o);
+    }
+  c->plain_comm.assign(inner.size(), {});
+  c->comm_levels.clear();
+  for (int l = 0; l < levels; ++l) {
+    ostc_fr_ctx_s::WgRange g;
+    g.lo = (int)wgs.size();
+    for (size_t q = 0; q < inner.size(); ++q)
+      if (inner[q].level == l) c->plain_comm[q] = append(inner[q].op);
+    g.n = (int)wgs.size() - g.lo;
+    c->comm_levels.push_back(g);
+  }
+  std::vector<FrBlockDev> hb;
+  for (auto& B : c->blocks) hb.push_back(B.d);
+  auto upload = [&](auto** to, const auto& h) {
+    void* v = nullptr;
+    if (h.empty()) return OSTC_OK;
+    FR_HIP(c, hipMalloc(&v, h.size() * sizeof(h[0])));
+    c->allocs.push_back(v);
+    FR_HIP(c, hipMemcpy(v, h.data(), h.size() * sizeof(h[0]), hipMemcpyHostToDevice));
+    *to = static_cast<std::remove_reference_t<decltype(*to)>>(v);
+    return OSTC_OK;
+  };
+  if (int r = upload(&c->d_blocks, hb)) return r;
+  if (int r = upload(&c->d_ghost, ops)) return r;
+  return upload(&c->d_ghost_wg, wgs);
+}
+
+void apply_bc(ostc_fr_ctx c, int b, long long* n) {
+  for (auto& w : c->plain_bc[b]) ghost(c, w, n);
+  if (c->inflow_noise) launch_count_pass(c->d_pass + b, 1, c->st, n);
+}
+
+void exchange(ostc_fr_ctx c, long long* n) {
+  for (auto& w : c->plain_comm) ghost(c, w, n);
 }
 
 // One SSP-RK3 step, src/RK.cuh:85-226 (MixtureModel::FR, laminar).
@@ -210,7 +331,7 @@ void step(ostc_fr_ctx c, long long* n, KernelTimer* tm) {
   if (c->sponge) {  // update_sponge_layer_value, then update_sponge_iter (src/RK.cuh:104-109)
     for (int b = 0; b < nb; ++b)
       if (c->blocks[b].d.sp_sigma) launch_sponge_mean(args(c, b), c->ns, c->d_sp_iter, c->st, n);
-    launch_count_pass(c->d_sp_iter, c->st, n);
+    launch_count_pass(c->d_sp_iter, 1, c->st, n);
   }
   for (int rk = 0; rk < 3; ++rk) {
     if (!c->s.fixed_time_step && rk == 0) {
@@ -231,8 +352,8 @@ void step(ostc_fr_ctx c, long long* n, KernelTimer* tm) {
 }
 
 // The same step with one launch per kernel kind over every block
-// (source, sweeps, update, properties, local dt); boundary conditions and
-// inner faces stay per face.  Each block's stage only reads and writes its
+// (source, sweeps, update, properties, local dt), per round of boundary
+// faces and per level of inner faces.  Each block's stage only reads and writes its
 // own arrays until the boundary conditions, so running all residuals, then
 // all updates, then all boundary conditions gives the per-block order's
 // result.
@@ -248,7 +369,7 @@ void step_batched(ostc_fr_ctx c, long long* n, KernelTimer* tm) {
   if (c->sponge) {
     for (int b = 0; b < nb; ++b)
       if (c->blocks[b].d.sp_sigma) launch_sponge_mean(h[b], c->ns, c->d_sp_iter, c->st, n);
-    launch_count_pass(c->d_sp_iter, c->st, n);
+    launch_count_pass(c->d_sp_iter, 1, c->st, n);
   }
   for (int rk = 0; rk < 3; ++rk) {
     if (!c->s.fixed_time_step && rk == 0) {
@@ -257,8 +378,9 @@ void step_batched(ostc_fr_ctx c, long long* n, KernelTimer* tm) {
     }
     launch_rhs_batched(h, nb, c->ns, c->st, n, tm);
     launch_update_batched(h, nb, c->ns, kRkA[rk], kRkB[rk], kRkC[rk], c->st, n, tm);
-    for (int b = 0; b < nb; ++b) apply_bc(c, b, n);
-    exchange(c, n);
+    for (auto& w : c->bc_rounds) ghost(c, w, n);
+    if (c->inflow_noise) launch_count_pass(c->d_pass, nb, c->st, n);
+    for (auto& w : c->comm_levels) ghost(c, w, n);
     launch_props_batched(h, nb, c->ns, c->st, n, tm);
   }
 }
@@ -732,6 +854,7 @@ int ostc_fr_finalize(ostc_fr_ctx c) {
   }
   c->h_args.clear();
   for (int b = 0; b < (int)c->blocks.size(); ++b) c->h_args.push_back(args(c, b));
+  if (int r = build_ghost(c)) return r;
   long long n = 0;
   launch_dt_set(c->d_dt, c->s.fixed_time_step ? c->s.dt : 1e6, c->st, &n);
   FR_HIP(c, hipEventCreate(&c->ev_a));

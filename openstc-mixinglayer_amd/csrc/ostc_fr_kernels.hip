@@ -305,9 +305,6 @@ __global__ __launch_bounds__(kT) void k_update_batched(FrBatch W, double ra, dou
   update_body<NS>(A, ra, rb, rc, w.x, w.y, w.z);
 }
 
-// apply_outflow / apply_periodic with scalars, src/BoundCond.cuh:205-233,
-// :1443-1486: one thread per face point over the face's padded tangential
-// extent, looping over the ngg ghost layers.
 // apply_farfield<FR>, src/BoundCond.cuh:755-1022, at face point ix: the
 // face point's normal Mach number (gamma from the property field) picks
 // supersonic inflow (the far field on the face point and its ghosts),
@@ -409,96 +406,135 @@ __device__ void farfield_point(const FrArgs& A, int axis, int side, const double
   }
 }
 
-template <int NS>
-__global__ __launch_bounds__(kT) void k_bc(FrArgs A, FaceBox fb, int type, const double* ff, const double* y,
-                                           const unsigned long long* pass) {
-  const FrBlockDev& B = A.B;
-  const int ext[3] = {B.mx, B.my, B.mz};
-  const int axis = fb.axis, side = fb.side;
-  const int q = blockIdx.x * kT + threadIdx.x;
-  if (q >= fb.n[0] * fb.n[1] * fb.n[2]) return;
-  int ix[3];
-  ix[0] = fb.lo[0] + q % fb.n[0];
-  ix[1] = fb.lo[1] + (q / fb.n[0]) % fb.n[1];
-  ix[2] = fb.lo[2] + q / (fb.n[0] * fb.n[1]);
-  if (type == 4) {
-    farfield_point<NS>(A, axis, side, ff, ix);
-    return;
-  }
-  if (type == 5) {  // apply_inflow, src/BoundCond.cuh:235-612
-    double st[6];
-    const bool upper = ostc::inflow_state(ff, y[q], *pass, ostc::inflow_point(axis, ix[0], ix[1], ix[2], B.mx, B.my, B.g), st);
-    const double* sv_in = ff + (upper ? ostc::kInflowSvUpper : ostc::kInflowSvLower);
-    const long long s = B.sz;
-    for (int g = 0; g <= B.g; ++g) {
-      int gi[3] = {ix[0], ix[1], ix[2]};
-      gi[axis] += g * side;
-      const long long pg = pid(B, gi[0], gi[1], gi[2]);
-#pragma unroll
-      for (int l = 0; l < 6; ++l) B.bv[pg + l * s] = st[l];
-#pragma unroll
-      for (int l = 0; l < NS; ++l) B.sv[pg + l * s] = sv_in[l];
-      cv_point<NS>(A, pg);
-    }
-    return;
-  }
-  int src[3] = {ix[0], ix[1], ix[2]};
-  if (type == 8) src[axis] = side < 0 ? ext[axis] - 1 : 0;
-  const long long s = B.sz;
-  for (int g = 1; g <= B.g; ++g) {
-    int gi[3] = {ix[0], ix[1], ix[2]}, si[3] = {src[0], src[1], src[2]};
-    gi[axis] += g * side;
-    if (type == 8) si[axis] += g * side;
-    const long long pg = pid(B, gi[0], gi[1], gi[2]), ps = pid(B, si[0], si[1], si[2]);
-#pragma unroll
-    for (int l = 0; l < 6; ++l) B.bv[pg + l * s] = B.bv[ps + l * s];
-#pragma unroll
-    for (int l = 0; l < NS; ++l) B.sv[pg + l * s] = B.sv[ps + l * s];
-    cv_point<NS>(A, pg);
-  }
+// Pointers into global memory: the block table is read from memory, so the
+// pointers it holds are generic to the compiler, and generic (flat) accesses
+// also wait on the LDS counter.
+template <class T>
+using gptr = __attribute__((address_space(1))) T*;
+
+struct NodeArrays {
+  gptr<double> bv, sv, cv;
+  long long s;
+};
+__device__ __forceinline__ NodeArrays node_arrays(const FrBlockDev& B) {
+  return NodeArrays{(gptr<double>)B.bv, (gptr<double>)B.sv, (gptr<double>)B.cv, B.sz};
 }
 
-// inner_communication with scalars, src/DataCommunication.cuh:60-105: the
-// shared node layer takes the mean of both blocks (in both), the ghost layers
-// the target's values.
 template <int NS>
-__global__ __launch_bounds__(kT) void k_comm(FrArgs A, FrBlockDev Tg, CommMap m) {
-  const FrBlockDev& B = A.B;
-  const long long q = (long long)blockIdx.x * kT + threadIdx.x;
-  if (q >= (long long)m.n[0] * m.n[1] * m.n[2]) return;
-  const int i = m.lo[0] + (int)(q % m.n[0]);
-  const int j = m.lo[1] + (int)((q / m.n[0]) % m.n[1]);
-  const int k = m.lo[2] + (int)(q / ((long long)m.n[0] * m.n[1]));
-  auto src_index = [&](int code) {
-    const int a = (code < 0 ? -code : code) - 1;
-    const int v = a == 0 ? i : (a == 1 ? j : k);
-    return code < 0 ? -v : v;
-  };
-  const int tx0 = m.off[0] + src_index(m.code[0]), tx1 = m.off[1] + src_index(m.code[1]),
-            tx2 = m.off[2] + src_index(m.code[2]);
-  const bool shared = (m.axis == 0 ? i : (m.axis == 1 ? j : k)) == m.shared;
-  const long long p = pid(B, i, j, k), pt = pid(Tg, tx0, tx1, tx2);
-  const long long s = B.sz, ts = Tg.sz;
-  if (shared) {
+struct Node { double q[6], Y[NS]; };
+
+template <int NS>
+__device__ __forceinline__ Node<NS> get_node(const NodeArrays& B, long long p) {
+  Node<NS> n;
 #pragma unroll
-    for (int l = 0; l < 6; ++l) {
-      const double ave{0.5 * (Tg.bv[pt + l * ts] + B.bv[p + l * s])};
-      B.bv[p + l * s] = ave;
-      Tg.bv[pt + l * ts] = ave;
-    }
+  for (int l = 0; l < 6; ++l) n.q[l] = B.bv[p + l * B.s];
 #pragma unroll
-    for (int l = 0; l < NS; ++l) {
-      const double ave{0.5 * (Tg.sv[pt + l * ts] + B.sv[p + l * s])};
-      B.sv[p + l * s] = ave;
-      Tg.sv[pt + l * ts] = ave;
-    }
-  } else {
+  for (int l = 0; l < NS; ++l) n.Y[l] = B.sv[p + l * B.s];
+  return n;
+}
+
+// The node's primitives and mass fractions and, from the same registers, its
+// cv (the values cv_point would compute after reading them back).
+template <int NS>
+__device__ __forceinline__ void put_node(const Tab* __restrict__ T, const NodeArrays& B, long long p,
+                                         const Node<NS>& n) {
+  const double rho = n.q[0];
+  const double e = total_energy<NS>(T, rho, n.q[1], n.q[2], n.q[3], n.q[4], n.q[5], n.Y);
 #pragma unroll
-    for (int l = 0; l < 6; ++l) B.bv[p + l * s] = Tg.bv[pt + l * ts];
+  for (int l = 0; l < 6; ++l) B.bv[p + l * B.s] = n.q[l];
 #pragma unroll
-    for (int l = 0; l < NS; ++l) B.sv[p + l * s] = Tg.sv[pt + l * ts];
+  for (int l = 0; l < NS; ++l) {
+    B.sv[p + l * B.s] = n.Y[l];
+    B.cv[p + (5 + l) * B.s] = rho * n.Y[l];
   }
-  cv_point<NS>(A, p);
+  B.cv[p] = rho;
+#pragma unroll
+  for (int d = 1; d < 4; ++d) B.cv[p + d * B.s] = rho * n.q[d];
+  B.cv[p + 4 * B.s] = e;
+}
+
+// Ghost-layer work of many faces in one launch: workgroup w runs 256 items of
+// one op, so the op and its blocks' descriptors are the same for the whole
+// workgroup and come by scalar loads.  Items: outflow and periodic faces
+// (apply_outflow, apply_periodic, src/BoundCond.cuh:205-233, :1443-1486) one
+// ghost node each; farfield and inflow faces (:755-1022, :235-612) one face
+// point with its ghost nodes; inner faces (inner_communication with scalars,
+// src/DataCommunication.cuh:60-105) one point of the face's box: the shared
+// node layer takes the mean of both blocks, in both, the ghost layers the
+// target's values.  Every item reads what it needs before its first store: a
+// chain of loads and stores that might alias took 41 us for a face of a few
+// thousand points (one launch per face; 8 us now).
+// FAR: the ops may hold farfield faces, whose iteration needs twice the
+// registers of everything else.
+template <int NS, bool FAR>
+__global__ __launch_bounds__(kT) void k_ghost(FrArgs A, const FrBlockDev* blocks, const GhostOp* ops,
+                                              const GhostWg* wgs) {
+  const GhostWg w = wgs[blockIdx.x];
+  const GhostOp& op = ops[w.op];
+  const int item = w.first + (int)threadIdx.x, pts = op.n[0] * op.n[1] * op.n[2];
+  if (item >= pts * op.layers) return;
+  const FrBlockDev& B = blocks[op.block];
+  const NodeArrays N = node_arrays(B);
+  const int layer = item / pts, t = item - layer * pts;
+  const int u = t / op.n[0], v = u / op.n[1];
+  const int i = op.lo[0] + t - u * op.n[0], j = op.lo[1] + u - v * op.n[1], k = op.lo[2] + v;
+  const int axis = op.axis, side = op.side;
+  const int di = axis == 0 ? side : 0, dj = axis == 1 ? side : 0, dk = axis == 2 ? side : 0;
+  switch (op.type) {
+    case GHOST_OUTFLOW: {
+      const int g = layer + 1;
+      put_node<NS>(A.T, N, pid(B, i + g * di, j + g * dj, k + g * dk), get_node<NS>(N, pid(B, i, j, k)));
+      break;
+    }
+    case GHOST_PERIODIC: {
+      const int g = layer + 1, m = axis == 0 ? B.mx : (axis == 1 ? B.my : B.mz), from = side < 0 ? m - 1 : 0;
+      const int si = axis == 0 ? from : i, sj = axis == 1 ? from : j, sk = axis == 2 ? from : k;
+      put_node<NS>(A.T, N, pid(B, i + g * di, j + g * dj, k + g * dk),
+                   get_node<NS>(N, pid(B, si + g * di, sj + g * dj, sk + g * dk)));
+      break;
+    }
+    case GHOST_INNER: {
+      const FrBlockDev& Tg = blocks[op.target];
+      const NodeArrays M = node_arrays(Tg);
+      auto src_index = [&](int code) {
+        const int a = (code < 0 ? -code : code) - 1;
+        const int x = a == 0 ? i : (a == 1 ? j : k);
+        return code < 0 ? -x : x;
+      };
+      const long long p = pid(B, i, j, k), pt = pid(Tg, op.off[0] + src_index(op.code[0]),
+                                                    op.off[1] + src_index(op.code[1]), op.off[2] + src_index(op.code[2]));
+      Node<NS> n = get_node<NS>(M, pt);
+      if ((axis == 0 ? i : (axis == 1 ? j : k)) == op.shared) {
+        const Node<NS> own = get_node<NS>(N, p);
+#pragma unroll
+        for (int l = 0; l < 6; ++l) n.q[l] = 0.5 * (n.q[l] + own.q[l]);
+#pragma unroll
+        for (int l = 0; l < NS; ++l) n.Y[l] = 0.5 * (n.Y[l] + own.Y[l]);
+#pragma unroll
+        for (int l = 0; l < 6; ++l) M.bv[pt + l * M.s] = n.q[l];
+#pragma unroll
+        for (int l = 0; l < NS; ++l) M.sv[pt + l * M.s] = n.Y[l];
+      }
+      put_node<NS>(A.T, N, p, n);
+      break;
+    }
+    case GHOST_INFLOW: {
+      Node<NS> n;
+      const bool upper = ostc::inflow_state(op.ff, op.y[t], *op.pass, ostc::inflow_point(axis, i, j, k, B.mx, B.my, B.g), n.q);
+      const double* sv_in = op.ff + (upper ? ostc::kInflowSvUpper : ostc::kInflowSvLower);
+#pragma unroll
+      for (int l = 0; l < NS; ++l) n.Y[l] = sv_in[l];
+      for (int g = 0; g <= B.g; ++g) put_node<NS>(A.T, N, pid(B, i + g * di, j + g * dj, k + g * dk), n);
+      break;
+    }
+    default:  // GHOST_FARFIELD
+      if constexpr (FAR) {
+        FrArgs F = A;
+        F.B = B;
+        const int ix[3] = {i, j, k};
+        farfield_point<NS>(F, axis, side, op.ff, ix);
+      }
+  }
 }
 
 // ------------------------------------------------------------ tile geometry
@@ -1496,21 +1532,25 @@ void launch_dt_set(double* dt, double v, hipStream_t st, long long* n) {
   ++*n;
 }
 
-void launch_bc(const FrArgs& A, int ns, const FaceBox& fb, int type, const double* ff, const double* y,
-               const unsigned long long* pass, hipStream_t st, long long* n) {
-  const long long cnt = (long long)fb.n[0] * fb.n[1] * fb.n[2];
-  OSTC_FR_DISPATCH(ns, hipLaunchKernelGGL(k_bc<NS>, dim3(nblk(cnt)), dim3(kT), 0, st, A, fb, type, ff, y, pass))
+void launch_ghost(const FrArgs& A, int ns, const FrBlockDev* blocks, const GhostOp* ops, const GhostWg* wgs, int n_wg,
+                  bool far, hipStream_t st, long long* n) {
+  if (n_wg <= 0) return;
+  if (far) {
+    OSTC_FR_DISPATCH(ns, hipLaunchKernelGGL((k_ghost<NS, true>), dim3(n_wg), dim3(kT), 0, st, A, blocks, ops, wgs))
+  } else {
+    OSTC_FR_DISPATCH(ns, hipLaunchKernelGGL((k_ghost<NS, false>), dim3(n_wg), dim3(kT), 0, st, A, blocks, ops, wgs))
+  }
   ++*n;
 }
 
-// One more boundary-condition pass of a block: the counter that keys the
+// One more boundary-condition pass of `count` blocks: the counters that key the
 // inflow's white noise (a kernel, so that a captured graph repeats it).
-__global__ void k_count_pass(unsigned long long* pass) {
-  if (threadIdx.x == 0) *pass += 1;
+__global__ void k_count_pass(unsigned long long* pass, int count) {
+  for (int b = threadIdx.x; b < count; b += 64) pass[b] += 1;
 }
 
-void launch_count_pass(unsigned long long* pass, hipStream_t st, long long* n) {
-  hipLaunchKernelGGL(k_count_pass, dim3(1), dim3(64), 0, st, pass);
+void launch_count_pass(unsigned long long* pass, int count, hipStream_t st, long long* n) {
+  hipLaunchKernelGGL(k_count_pass, dim3(1), dim3(64), 0, st, pass, count);
   ++*n;
 }
 
@@ -1530,12 +1570,6 @@ __global__ __launch_bounds__(kT) void k_sponge_mean(FrBlockDev B, const unsigned
 
 void launch_sponge_mean(const FrArgs& A, int ns, const unsigned long long* iter, hipStream_t st, long long* n) {
   OSTC_FR_DISPATCH(ns, hipLaunchKernelGGL(k_sponge_mean<NS>, dim3(nblk(A.B.n0)), dim3(kT), 0, st, A.B, iter))
-  ++*n;
-}
-
-void launch_comm(const FrArgs& A, const FrBlockDev& Tg, int ns, const CommMap& m, hipStream_t st, long long* n) {
-  const long long cnt = (long long)m.n[0] * m.n[1] * m.n[2];
-  OSTC_FR_DISPATCH(ns, hipLaunchKernelGGL(k_comm<NS>, dim3(nblk(cnt)), dim3(kT), 0, st, A, Tg, m))
   ++*n;
 }
 
