@@ -4,7 +4,13 @@ workgroups (a partial last one), farfield and other faces in the same round,
 inner faces whose edges conflict.  Against the oracle's sequential faces,
 primitives and mass fractions <= 1e-9 after two steps (the bound of the
 temperature iteration's stop, as in the other step tests), and the per-block
-launches of the same ops bit for bit."""
+launches of the same ops bit for bit.
+
+Periodic axes have at least 5 cells: on 4, the five points of a WENO-Z5 stencil
+begin and end with the same node, beta_0 - beta_2 is a rounding error wherever
+the three others agree, and the weights, tau / (eps + beta_1)^2 up to
+(2^-53 / 1e-20)^2 = 1e8, are that error's (measured 2e-5 of w between two orders
+of summation)."""
 import numpy as np
 import pytest
 
@@ -17,7 +23,7 @@ pytestmark = pytest.mark.gpu
 MX = pkg.mixture
 
 
-@pytest.mark.parametrize("cells,y_bc,spatial", [(([4, 5], [4], [4, 6]), 4, False), (([4], [5, 4], [4]), 6, True),
+@pytest.mark.parametrize("cells,y_bc,spatial", [(([4, 5], [4], [4, 6]), 4, False), (([4], [5, 4], [5]), 6, True),
                                                 (([20, 4], [5, 17], [4, 5]), 4, True)],
                          ids=["farfield-temporal", "outflow-spatial", "farfield-spatial"])
 def test_ghost_rounds_and_levels(cells, y_bc, spatial):
