@@ -57,7 +57,6 @@ struct ostc_fr_ctx_s {
   ostc_fr_setup s{};
   ostc_mech_tables tab{};
   Tab* d_tab = nullptr;
-  double* d_tlog = nullptr;        // log tables of the transport kernel (16 + 256 doubles)
   int ns = 0, nv = 5, ngg = 3;
   hipStream_t st = nullptr;
   bool own_stream = false;
@@ -136,7 +135,6 @@ FrArgs args(ostc_fr_ctx c, int b) {
   FrArgs a{};
   a.B = c->blocks[b].d;
   a.T = c->d_tab;
-  a.tlog = c->d_tlog;
   a.scheme = c->s.inviscid_scheme;
   a.viscous = c->s.viscous_order != 0;
   a.reaction = c->s.reaction != 0;
@@ -157,6 +155,42 @@ int check_ready(ostc_fr_ctx c) {
   if (!c) return OSTC_ERR_ARG;
   if (!c->finalized) return fail(c, OSTC_ERR_STATE, "context not finalized");
   return OSTC_OK;
+}
+
+Tab derive_tables(const ostc_mech_tables& m) {
+  Tab t{};
+  static_cast<ostc_mech_tables&>(t) = m;
+  t.mid_lo = t.mid_hi = m.t_mid[0];
+  for (int i = 0; i < m.n_spec; ++i) {
+    t.imw[i] = 1.0 / m.mw[i];
+    t.r[i] = kRu / m.mw[i];
+    t.mid_lo = std::min(t.mid_lo, m.t_mid[i]);
+    t.mid_hi = std::max(t.mid_hi, m.t_mid[i]);
+    t.low_max = std::max(t.low_max, m.t_low[i]);
+    for (int side = 0; side < 2; ++side) {
+      const double* c = side ? m.high_coeff[i] : m.low_coeff[i];
+      for (int k = 0; k < 5; ++k) {
+        t.cpp[side][i][k] = c[k] * t.r[i];
+        t.hp[side][i][k] = c[k] * t.r[i] / (k + 1);
+      }
+      t.hp[side][i][5] = c[5] * t.r[i];
+      const double f[7] = {1.0, -1.0 / 2, -1.0 / 6, -1.0 / 12, -1.0 / 20, 1.0, -1.0};
+      for (int k = 0; k < 7; ++k) t.gp[side][i][k] = c[k] * f[k];
+    }
+    t.vis_k[i] = std::pow(m.lj_potent_inv[i], -0.145);
+    for (int n = 0; n < m.n_spec; ++n)
+      if (n != i) {
+        t.dif_k[i][n] = std::pow(m.kb_over_eps_jk[i][n], -0.145);
+        t.inv_bin[i][n] = 1.0 / m.binary_diffusivity_coeff[i][n];
+      }
+  }
+  for (int q = 0; q < m.n_reac; ++q) {
+    // equilibrium kb is used only if some reaction is neither irreversible nor
+    // REV (src/FiniteRateChem.cu:110-128)
+    if (m.label[q] != 0 && m.rev_type[q] != 1) t.use_kc = 1;
+    for (int i = 0; i < m.n_spec; ++i) t.dnu[q][i] = m.stoi_b[q][i] - m.stoi_f[q][i];
+  }
+  return t;
 }
 
 // src/BoundCond.cuh:1488-1678: farfield, outflow, inflow, ..., periodic
@@ -766,18 +800,9 @@ int ostc_fr_finalize(ostc_fr_ctx c) {
   if (c->finalized) return OSTC_OK;
   if (c->blocks.empty()) return fail(c, OSTC_ERR_STATE, "no blocks");
   FR_HIP(c, hipMalloc((void**)&c->d_tab, sizeof(Tab)));
-  FR_HIP(c, hipMemcpyAsync(c->d_tab, &c->tab, sizeof(Tab), hipMemcpyHostToDevice, c->st));
   {
-    // logarithms of the temperature scales of the collision integrals
-    static_assert(OSTC_MAX_SPEC == 16, "log table layout");
-    std::vector<double> h(16 + 16 * 16, 0.0);  // the copy below completes before h goes out of scope
-    for (int l = 0; l < c->ns; ++l) h[l] = std::log(c->tab.lj_potent_inv[l]);
-    for (int m = 0; m < c->ns; ++m)
-      for (int n = 0; n < c->ns; ++n)
-        if (m != n) h[16 + 16 * m + n] = std::log(c->tab.kb_over_eps_jk[m][n]);
-    if (int r = dalloc(c, &c->d_tlog, h.size())) return r;
-    FR_HIP(c, hipMemcpyAsync(c->d_tlog, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice, c->st));
-    FR_HIP(c, hipStreamSynchronize(c->st));
+    const Tab t = derive_tables(c->tab);
+    FR_HIP(c, hipMemcpy(c->d_tab, &t, sizeof(Tab), hipMemcpyHostToDevice));
   }
   const int g = c->ngg, nv = c->nv, ns = c->ns;
   for (auto& h : c->blocks) {

@@ -134,9 +134,9 @@ __device__ __forceinline__ void props_body(const FrArgs& A, const int wx, const 
 #pragma unroll
   for (int l = 0; l < NS; ++l) {
     Y[l] = B.sv[p + l * s];
-    mw += Y[l] / A.T->mw[l];
+    mw += Y[l] * A.T->imw[l];
     cp_tot += Y[l] * cp[l];
-    cvv += Y[l] * (cp[l] - kRu / A.T->mw[l]);
+    cvv += Y[l] * (cp[l] - A.T->r[l]);
   }
   mw = 1 / mw;
   const double gam = cp_tot / cvv;
@@ -145,7 +145,7 @@ __device__ __forceinline__ void props_body(const FrArgs& A, const int wx, const 
   B.gam[p] = gam;
   B.cc[p] = c;
   double mu, lam, rd[NS];
-  transport<NS>(A.T, A.tlog, t, B.bv[p + 4 * s], B.bv[p], Y, mw, cp, &mu, &lam, rd);
+  transport<NS>(A.T, t, B.bv[p + 4 * s], B.bv[p], Y, mw, cp, &mu, &lam, rd);
   B.mul[p] = mu;
   B.lam[p] = lam;
 #pragma unroll
@@ -285,7 +285,7 @@ __device__ __forceinline__ void update_body(const FrArgs& A, double ra, double r
     B.sv[p + l * s] = Y[l];
   }
 #pragma unroll
-  for (int l = 0; l < NS; ++l) mw += Y[l] / A.T->mw[l];
+  for (int l = 0; l < NS; ++l) mw += Y[l] * A.T->imw[l];
   mw = 1 / mw;
   const double gas_const = kRu / mw;
   const double e = cv[4] / cv[0] - 0.5 * (u * u + v * v + w * w);
@@ -331,7 +331,7 @@ __device__ void farfield_point(const FrArgs& A, int axis, int side, const double
   const double gamma_b = B.gam[p];
   double mw_inv{0};
 #pragma unroll
-  for (int l = 0; l < NS; ++l) mw_inv += sv_b[l] / A.T->mw[l];
+  for (int l = 0; l < NS; ++l) mw_inv += sv_b[l] * A.T->imw[l];
   double mw = 1.0 / mw_inv;
   const double p_b = B.bv[p + 4 * s], rho_b = B.bv[p];
   const double a_b = sqrt(gamma_b * p_b / rho_b);
@@ -1227,8 +1227,8 @@ __device__ __forceinline__ void viscous_body(const FrArgs& A, const int wx, cons
       const double gy = kx * y_x + ky * y_y + kz * y_z;
       ddf[l] = gy;
       corr += diffusivity[l] * gy;
-      sum_grad_over_w += gy / A.T->mw[l];
-      mw_tot += yk[l] / A.T->mw[l];
+      sum_grad_over_w += gy * A.T->imw[l];
+      mw_tot += yk[l] * A.T->imw[l];
       sum_rhoDkYk += diffusivity[l] * yk[l];
     }
     mw_tot = 1.0 / mw_tot;
@@ -1242,8 +1242,8 @@ __device__ __forceinline__ void viscous_body(const FrArgs& A, const int wx, cons
       const double gp = (kx * p_x + ky * p_y + kz * p_z) / (0.5 * (B.bv[p1 + 4 * s] + B.bv[p + 4 * s]));
 #pragma unroll
       for (int l = 0; l < NS; ++l) {
-        ddf[l] += (mw_tot / A.T->mw[l] - 1) * yk[l] * gp;
-        corr += (mw_tot / A.T->mw[l] - 1) * yk[l] * gp * diffusivity[l];
+        ddf[l] += (mw_tot * A.T->imw[l] - 1) * yk[l] * gp;
+        corr += (mw_tot * A.T->imw[l] - 1) * yk[l] * gp * diffusivity[l];
       }
     }
     double h[NS];
