@@ -169,11 +169,8 @@ Tab derive_tables(const ostc_mech_tables& m) {
     t.low_max = std::max(t.low_max, m.t_low[i]);
     for (int side = 0; side < 2; ++side) {
       const double* c = side ? m.high_coeff[i] : m.low_coeff[i];
-      for (int k = 0; k < 5; ++k) {
-        t.cpp[side][i][k] = c[k] * t.r[i];
-        t.hp[side][i][k] = c[k] * t.r[i] / (k + 1);
-      }
-      t.hp[side][i][5] = c[5] * t.r[i];
+      for (int k = 0; k < 5; ++k) t.cpp[side][i][k] = c[k] * t.r[i];
+      t.h0[side][i] = c[5] * t.r[i];
       const double f[7] = {1.0, -1.0 / 2, -1.0 / 6, -1.0 / 12, -1.0 / 20, 1.0, -1.0};
       for (int k = 0; k < 7; ++k) t.gp[side][i][k] = c[k] * f[k];
     }

@@ -30,7 +30,7 @@ struct Tab : ostc_mech_tables {
   double imw[OSTC_MAX_SPEC], r[OSTC_MAX_SPEC];  // 1 / W, R_u / W
   double mid_lo, mid_hi, low_max;               // least and largest t_mid, largest t_low
   double cpp[2][OSTC_MAX_SPEC][5];              // cp = sum cpp[k] t^k; [0] low range, [1] high range
-  double hp[2][OSTC_MAX_SPEC][6];               // h = hp[5] + sum hp[k] t^(k+1)
+  double h0[2][OSTC_MAX_SPEC];                  // h = h0 + sum cpp[k] t^(k+1) / (k+1)
   double gp[2][OSTC_MAX_SPEC][7];               // g/RT = gp[0] (1 - log t) + sum_1..4 gp[k] t^k + gp[5]/t + gp[6]
   double vis_k[OSTC_MAX_SPEC];                  // lj_potent_inv^-0.145
   double dif_k[OSTC_MAX_SPEC][OSTC_MAX_SPEC];   // kb_over_eps_jk^-0.145
@@ -65,11 +65,30 @@ __device__ __forceinline__ double poly_h(const double* c, double t) {
   return __builtin_fma(t, poly_cp(c, t), c[5]);
 }
 
+// One species' enthalpy and heat capacity in the reference's operation order
+// and rounding: what the face decomposition reads has to match it bit by bit
+// (see char_face).  The quotients are the shorter sequences of div64 with the
+// same result.
+__device__ __forceinline__ double species_cp(const double* c, double t) {
+  const double t2 = t * t, t3 = t2 * t, t4 = t3 * t;
+  return c[0] + c[1] * t + c[2] * t2 + c[3] * t3 + c[4] * t4;
+}
+__device__ __forceinline__ double species_h(const double* c, double t) {
+  const double t2 = t * t, t3 = t2 * t, t4 = t3 * t, t5 = t4 * t;
+  return c[0] * t + 0.5 * c[1] * t2 + div64(c[2] * t3, 3.0, 1.0 / 3.0) + 0.25 * c[3] * t4 + 0.2 * c[4] * t5 + c[5];
+}
+__device__ __forceinline__ const double* coefficients(const Tab* __restrict__ T, int i, int side) {
+  return side ? T->high_coeff[i] : T->low_coeff[i];
+}
+
 // compute_enthalpy (Combustion2Part), src/Thermo.cu:130-148
 template <int NS>
 __device__ __forceinline__ void enthalpy(const Tab* __restrict__ T, double t, double* h) {
   each_species<NS>(T, t, [&](int i, int side, double tt) {
-    h[i] = __builtin_fma(poly_cp(T->cpp[side][i], tt), t - tt, poly_h(T->hp[side][i], tt));
+    const double* c = coefficients(T, i, side);
+    double v = species_h(c, tt);
+    if (t < T->t_low[i]) v += species_cp(c, tt) * (t - tt);
+    h[i] = v * T->r[i];
   });
 }
 
@@ -77,15 +96,21 @@ __device__ __forceinline__ void enthalpy(const Tab* __restrict__ T, double t, do
 template <int NS>
 __device__ __forceinline__ void enthalpy_cp(const Tab* __restrict__ T, double t, double* h, double* cp) {
   each_species<NS>(T, t, [&](int i, int side, double tt) {
-    cp[i] = poly_cp(T->cpp[side][i], tt);
-    h[i] = __builtin_fma(cp[i], t - tt, poly_h(T->hp[side][i], tt));
+    const double* c = coefficients(T, i, side);
+    const double k = species_cp(c, tt);
+    double v = species_h(c, tt);
+    if (t < T->t_low[i]) v += k * (t - tt);
+    h[i] = v * T->r[i];
+    cp[i] = k * T->r[i];
   });
 }
 
 // compute_cp (Combustion2Part), src/Thermo.cu:174-188
 template <int NS>
 __device__ __forceinline__ void heat_capacity(const Tab* __restrict__ T, double t, double* cp) {
-  each_species<NS>(T, t, [&](int i, int side, double tt) { cp[i] = poly_cp(T->cpp[side][i], tt); });
+  each_species<NS>(T, t, [&](int i, int side, double tt) {
+    cp[i] = species_cp(coefficients(T, i, side), tt) * T->r[i];
+  });
 }
 
 // compute_gibbs_div_rt (Combustion2Part), src/Thermo.cu:190-208
@@ -292,7 +317,7 @@ __device__ __forceinline__ double temperature(const Tab* __restrict__ T, double 
     for (int i = 0; i < NS; ++i) {
 #pragma unroll
       for (int k = 0; k < 5; ++k) mc[k] = __builtin_fma(Y[i], T->cpp[side][i][k], mc[k]);
-      mh[5] = __builtin_fma(Y[i], T->hp[side][i][5], mh[5]);
+      mh[5] = __builtin_fma(Y[i], T->h0[side][i], mh[5]);
     }
     constexpr double inv[5]{1.0, 1.0 / 2, 1.0 / 3, 1.0 / 4, 1.0 / 5};
 #pragma unroll

@@ -134,7 +134,7 @@ __device__ __forceinline__ void props_body(const FrArgs& A, const int wx, const 
 #pragma unroll
   for (int l = 0; l < NS; ++l) {
     Y[l] = B.sv[p + l * s];
-    mw += Y[l] * A.T->imw[l];
+    mw += div64(Y[l], A.T->mw[l], A.T->imw[l]);
     cp_tot += Y[l] * cp[l];
     cvv += Y[l] * (cp[l] - A.T->r[l]);
   }
@@ -285,7 +285,7 @@ __device__ __forceinline__ void update_body(const FrArgs& A, double ra, double r
     B.sv[p + l * s] = Y[l];
   }
 #pragma unroll
-  for (int l = 0; l < NS; ++l) mw += Y[l] * A.T->imw[l];
+  for (int l = 0; l < NS; ++l) mw += div64(Y[l], A.T->mw[l], A.T->imw[l]);
   mw = 1 / mw;
   const double gas_const = kRu / mw;
   const double e = cv[4] / cv[0] - 0.5 * (u * u + v * v + w * w);
@@ -573,6 +573,16 @@ __device__ __forceinline__ int face_slot(int col, int f) {
   return DIR == 0 ? col * F + f : f * TW + col;
 }
 
+// LDS slot of point sp of column col among a tile's split fluxes, with
+// consecutive lanes on consecutive slots as for the face fluxes; the points of
+// a stencil are point_step apart.
+template <int DIR, int TW, int P>
+__device__ __forceinline__ int point_slot(int col, int sp) {
+  return DIR == 0 ? col * P + sp : sp * TW + col;
+}
+template <int DIR, int TW>
+constexpr int point_step() { return DIR == 0 ? 1 : TW; }
+
 // Positivity-preserving limiter on the species part of one face,
 // src/WENO.cu:1538-1580.
 template <int NS>
@@ -634,7 +644,7 @@ __device__ __forceinline__ void split_fluxes(const FrArgs& A, double* Fp, double
     const int t = t0 - G - LEFT + sp;
     int idx[3];
     tile_idx<DIR>(col0, t < -G ? -G : t, col, third, idx);
-    const int slot = col * P + sp;
+    const int slot = point_slot<DIR, TW, P>(col, sp);
     if (idx[across] < ext[across] && t < m + G) {
       const long long p = pid(B, idx[0], idx[1], idx[2]);
       double q[NV + 2], kk[3];
@@ -646,24 +656,15 @@ __device__ __forceinline__ void split_fluxes(const FrArgs& A, double* Fp, double
       for (int c = 0; c < 3; ++c) kk[c] = B.met[p + (3 * DIR + c) * s];
       const double jac = B.jac[p];
       // compute_flux, src/WENO.cu:697-720
-      const double Uk{(q[1] * kk[0] + q[2] * kk[1] + q[3] * kk[2]) / q[0]};
+      const double Uk{div64(q[1] * kk[0] + q[2] * kk[1] + q[3] * kk[2], q[0])};
       const double pk{q[NV]};
       const double cGradK = q[NV + 1] * sqrt(kk[0] * kk[0] + kk[1] * kk[1] + kk[2] * kk[2]);
-      const double lambda0 = fabs(Uk) + cGradK;
-      Fp[0 * NP + slot] = 0.5 * jac * (Uk * q[0] + lambda0 * q[0]);
-      Fp[1 * NP + slot] = 0.5 * jac * (Uk * q[1] + pk * kk[0] + lambda0 * q[1]);
-      Fp[2 * NP + slot] = 0.5 * jac * (Uk * q[2] + pk * kk[1] + lambda0 * q[2]);
-      Fp[3 * NP + slot] = 0.5 * jac * (Uk * q[3] + pk * kk[2] + lambda0 * q[3]);
-      Fp[4 * NP + slot] = 0.5 * jac * (Uk * (q[4] + pk) + lambda0 * q[4]);
-      Fm[0 * NP + slot] = 0.5 * jac * (Uk * q[0] - lambda0 * q[0]);
-      Fm[1 * NP + slot] = 0.5 * jac * (Uk * q[1] + pk * kk[0] - lambda0 * q[1]);
-      Fm[2 * NP + slot] = 0.5 * jac * (Uk * q[2] + pk * kk[1] - lambda0 * q[2]);
-      Fm[3 * NP + slot] = 0.5 * jac * (Uk * q[3] + pk * kk[2] - lambda0 * q[3]);
-      Fm[4 * NP + slot] = 0.5 * jac * (Uk * (q[4] + pk) - lambda0 * q[4]);
+      const double lambda0 = fabs(Uk) + cGradK, hj = 0.5 * jac;
 #pragma unroll
-      for (int l = 5; l < NV; ++l) {
-        Fp[l * NP + slot] = 0.5 * jac * (Uk * q[l] + lambda0 * q[l]);
-        Fm[l * NP + slot] = 0.5 * jac * (Uk * q[l] - lambda0 * q[l]);
+      for (int l = 0; l < NV; ++l) {
+        const double f = l >= 1 && l <= 3 ? Uk * q[l] + pk * kk[l - 1] : (l == 4 ? Uk * (q[4] + pk) : Uk * q[l]);
+        Fp[l * NP + slot] = hj * (f + lambda0 * q[l]);
+        Fm[l * NP + slot] = hj * (f - lambda0 * q[l]);
       }
     } else {
 #pragma unroll
@@ -710,7 +711,8 @@ __device__ __forceinline__ void inviscid_body(const FrArgs& A, const int wx, con
   const bool active = idx[across] < ext[across] && tl < m;
   double fc[NV];
   if (active) {
-    const int sl = col * P + (f + G - 1);  // LDS slot of the left cell
+    constexpr int PS = point_step<DIR, TW>();
+    const int sl = point_slot<DIR, TW, P>(col, f + G - 1);  // LDS slot of the left cell
     const long long pl = pid(B, idx[0], idx[1], idx[2]);
     int idr[3] = {idx[0], idx[1], idx[2]};
     idr[DIR] += 1;
@@ -735,7 +737,7 @@ __device__ __forceinline__ void inviscid_body(const FrArgs& A, const int wx, con
       eps_scaled[2] = eps_scaled[1] * A.v_ref * A.v_ref;
       if (A.pp) {
 #pragma unroll
-        for (int l = 0; l < NS; ++l) f1[l] = 0.5 * Fp[(l + 5) * NP + sl] + 0.5 * Fm[(l + 5) * NP + sl + 1];
+        for (int l = 0; l < NS; ++l) f1[l] = 0.5 * Fp[(l + 5) * NP + sl] + 0.5 * Fm[(l + 5) * NP + sl + PS];
       }
 #pragma unroll
       for (int l = 0; l < NV; ++l) {
@@ -743,8 +745,8 @@ __device__ __forceinline__ void inviscid_body(const FrArgs& A, const int wx, con
         double vp[W], vm[W];
 #pragma unroll
         for (int r = 0; r < W; ++r) {
-          vp[r] = Fp[l * NP + sl - W / 2 + r];
-          vm[r] = Fm[l * NP + sl - W / 2 + 1 + r];
+          vp[r] = Fp[l * NP + sl + (r - W / 2) * PS];
+          vm[r] = Fm[l * NP + sl + (r - W / 2 + 1) * PS];
         }
         if constexpr (W == 7) fc[l] = weno7z(vp, vm, eh);  // compute_weno_flux_cp, 71 (src/WENO.cu:1516-1534)
         else fc[l] = weno5z(vp, vm, eh);
@@ -806,6 +808,13 @@ template <> struct TileCh<2> { static constexpr int TW = 8, F = 16; };
 // limiter), each in the reference's term order, so the face flux is the
 // same as one thread computing every field.  Both halves form the face's Roe
 // state themselves.
+// FP64 issue bounds it (3000 instructions a thread, 43 % of the time at the
+// full rate), then latency: the 54 KB of split fluxes let three workgroups
+// share a CU, so the registers are held to a third of the file as well.  The
+// projections run unrolled over the stencil with one point's sums finished
+// before the next point's loads (without that 296 registers, one wave a SIMD),
+// and what only the limiter needs is loaded where it runs.  256x128x64: a
+// sweep 0.95-1.07 -> 0.65-0.69 ms.
 template <int DIR, int NS, int SCHEME>
 __device__ __forceinline__ void inviscid_ch_body(const FrArgs& A, const int wx, const int wy, const int wz) {
   constexpr int G = SCHEME == 72 ? 4 : 3, W = 2 * G - 1;
@@ -843,8 +852,8 @@ __device__ __forceinline__ void inviscid_ch_body(const FrArgs& A, const int wx, 
   double fc[NV];
   CharFace<NS> C;
   long long pl = 0, pr = 0;
-  double jac1 = 0, jac2 = 0, f1[NS];
-  const int sl = col * P + (f + G - 1 + LEFT);  // LDS slot of the left cell
+  constexpr int PS = point_step<DIR, TW>();
+  const int sl = point_slot<DIR, TW, P>(col, f + G - 1 + LEFT);  // LDS slot of the left cell
   if (active) {
     pl = pid(B, idx[0], idx[1], idx[2]);
     int idr[3] = {idx[0], idx[1], idx[2]};
@@ -856,8 +865,7 @@ __device__ __forceinline__ void inviscid_ch_body(const FrArgs& A, const int wx, 
       ml[c] = B.met[pl + (3 * DIR + c) * s];
       mr[c] = B.met[pr + (3 * DIR + c) * s];
     }
-    jac1 = B.jac[pl];
-    jac2 = B.jac[pr];
+    const double jac1 = B.jac[pl], jac2 = B.jac[pr];
     {
       double cvl[NV + 2], cvr[NV + 2];
 #pragma unroll
@@ -870,44 +878,38 @@ __device__ __forceinline__ void inviscid_ch_body(const FrArgs& A, const int wx, 
       cvl[NV + 1] = B.cc[pl];
       cvr[NV + 1] = B.cc[pr];
       char_face<NS>(A.T, cvl, cvr, ml, mr, jac1, jac2, C);
-      if (A.pp && half == 1) {
-        const double srThis = fabs((ml[0] * cvl[1] + ml[1] * cvl[2] + ml[2] * cvl[3]) / cvl[0] +
-                                   cvl[NV + 1] * sqrt(ml[0] * ml[0] + ml[1] * ml[1] + ml[2] * ml[2]));
-        const double srNext = fabs((mr[0] * cvr[1] + mr[1] * cvr[2] + mr[2] * cvr[3]) / cvr[0] +
-                                   cvr[NV + 1] * sqrt(mr[0] * mr[0] + mr[1] * mr[1] + mr[2] * mr[2]));
-#pragma unroll
-        for (int l = 0; l < NS; ++l)
-          f1[l] = 0.5 * (Fp[(l + 5) * NP + sl] + srThis * cvl[l + 5] * jac1) +
-                  0.5 * (Fp[(l + 5) * NP + sl + 1] - srNext * cvr[l + 5] * jac2);
-      }
     }
     constexpr double eps{1e-40};
     const double eps_scaled = eps * A.weno_eps_scale * 0.25 * (C.nj[0] * C.nj[0] + C.nj[1] * C.nj[1] + C.nj[2] * C.nj[2]);
+    auto point = [&](const double* F, int n, int at) { return F[n * NP + sl + at * PS]; };
     // acoustic and entropy fields of this half
     const int l_lo = half == 0 ? 0 : 3, l_hi = half == 0 ? 3 : 5;
 #pragma unroll 1
     for (int l = l_lo; l < l_hi; ++l) {
       double L[5];
       const double cas = char_row<NS>(C, l, L);
-      double vPlus[W], vMinus[W];
-#pragma unroll 1
-      for (int r = 0; r < W; ++r) {
-        double ap = 0, am = 0;
+      double vPlus[W], vMinus[W], K[NS];
 #pragma unroll
-        for (int n = 0; n < 5; ++n) {
-          ap += L[n] * Fp[n * NP + sl - W / 2 + r - sh];
-          am += L[n] * Fm[n * NP + sl - W / 2 + 1 + r - sh];
+      for (int n = 0; n < NS; ++n) K[n] = cas * C.coupling[n];
+#pragma unroll
+      for (int r = 0; r < W; ++r) {
+        double ap = L[0] * point(Fp, 0, r - W / 2 - sh), am = L[0] * point(Fm, 0, r - W / 2 + 1 - sh);
+#pragma unroll
+        for (int n = 1; n < 5; ++n) {
+          ap += L[n] * point(Fp, n, r - W / 2 - sh);
+          am += L[n] * point(Fm, n, r - W / 2 + 1 - sh);
         }
 #pragma unroll
         for (int n = 0; n < NS; ++n) {
-          ap += cas * C.coupling[n] * Fp[(5 + n) * NP + sl - W / 2 + r];
-          am += cas * C.coupling[n] * Fm[(5 + n) * NP + sl - W / 2 + 1 + r];
+          ap += K[n] * point(Fp, 5 + n, r - W / 2);
+          am += K[n] * point(Fm, 5 + n, r - W / 2 + 1);
         }
-#pragma unroll
-        for (int qq = 0; qq < W; ++qq) {
-          vPlus[qq] = (qq == r) ? ap : vPlus[qq];
-          vMinus[qq] = (qq == r) ? am : vMinus[qq];
-        }
+        // one point's loads and sums at a time: left to itself the scheduler
+        // hoists the 140 loads of all five
+        asm volatile("" : "+v"(ap), "+v"(am)::"memory");
+        __builtin_amdgcn_sched_barrier(0);
+        vPlus[r] = ap;
+        vMinus[r] = am;
       }
       double v;
       if constexpr (W == 7) v = weno7z(vPlus, vMinus, eps_scaled);
@@ -922,12 +924,14 @@ __device__ __forceinline__ void inviscid_ch_body(const FrArgs& A, const int wx, 
       const double y = C.y[l];
 #pragma unroll
       for (int r = 0; r < W; ++r) {
-        vPlus[r] = -y * Fp[sl - W / 2 + r] + Fp[(5 + l) * NP + sl - W / 2 + r];
-        vMinus[r] = -y * Fm[sl - W / 2 + 1 + r] + Fm[(5 + l) * NP + sl - W / 2 + 1 + r];
+        vPlus[r] = -y * point(Fp, 0, r - W / 2) + point(Fp, 5 + l, r - W / 2);
+        vMinus[r] = -y * point(Fm, 0, r - W / 2 + 1) + point(Fm, 5 + l, r - W / 2 + 1);
       }
       double v;
       if constexpr (W == 7) v = weno7z(vPlus, vMinus, eps_scaled);
       else v = weno5z(vPlus, vMinus, eps_scaled);
+      asm volatile("" : "+v"(v)::"memory");
+      __builtin_amdgcn_sched_barrier(0);
       fch[(5 + l) * NF + q] = v;
     }
   }
@@ -958,16 +962,26 @@ __device__ __forceinline__ void inviscid_ch_body(const FrArgs& A, const int wx, 
       fc[1] = f[1];
       fc[2] = f[2];
       fc[3] = f[3];
-      fc[4] = f[4] - add * C.c * C.c / C.gm1;
+      fc[4] = f[4] - div64(add * C.c * C.c, C.gm1);
     } else {
 #pragma unroll
       for (int l = 0; l < NS; ++l) fc[5 + l] = C.y[l] * f0 + fch[(5 + l) * NF + q];
       if (A.pp) {
-        double ql[NS], qr[NS];
+        // the first-order flux from each side's spectral radius
+        auto radius = [&](long long p) {
+          const double k0 = B.met[p + (3 * DIR) * s], k1 = B.met[p + (3 * DIR + 1) * s], k2 = B.met[p + (3 * DIR + 2) * s];
+          return fabs((k0 * B.cv[p + s] + k1 * B.cv[p + 2 * s] + k2 * B.cv[p + 3 * s]) / B.cv[p] +
+                      B.cc[p] * sqrt(k0 * k0 + k1 * k1 + k2 * k2));
+        };
+        const double srThis = radius(pl), srNext = radius(pr);
+        const double jac1 = B.jac[pl], jac2 = B.jac[pr];
+        double ql[NS], qr[NS], f1[NS];
 #pragma unroll
         for (int l = 0; l < NS; ++l) {
           ql[l] = B.cv[pl + (5 + l) * s];
           qr[l] = B.cv[pr + (5 + l) * s];
+          f1[l] = 0.5 * (Fp[(l + 5) * NP + sl] + srThis * ql[l] * jac1) +
+                  0.5 * (Fp[(l + 5) * NP + sl + PS] - srNext * qr[l] * jac2);
         }
         pp_limit<NS>(fc + 5, f1, ql, qr, jac1, jac2, *A.dt, tl, m);
       }
@@ -992,11 +1006,11 @@ __device__ __forceinline__ void inviscid_ch_body(const FrArgs& A, const int wx, 
   }
 }
 template <int DIR, int NS, int SCHEME>
-__global__ __launch_bounds__(kT) void k_inviscid_ch(FrArgs A) {
+__global__ __launch_bounds__(kT, 3) void k_inviscid_ch(FrArgs A) {
   inviscid_ch_body<DIR, NS, SCHEME>(A, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 template <int DIR, int NS, int SCHEME>
-__global__ __launch_bounds__(kT) void k_inviscid_ch_batched(FrBatch W) {
+__global__ __launch_bounds__(kT, 3) void k_inviscid_ch_batched(FrBatch W) {
   const WgPos w = wg_pos(W);
   FrArgs A = W.common;
   A.B = W.blocks[w.b];

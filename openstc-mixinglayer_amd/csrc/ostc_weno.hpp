@@ -48,6 +48,25 @@ __device__ __forceinline__ double sqrt64(double x) {
   return __builtin_fma(__builtin_fma(-h1, h1, x), g1, h1);
 }
 
+// n / d as an IEEE division rounds it, for operands and quotient of ordinary
+// magnitude: the compiler's own sequence for a division without its scaling,
+// fix-up and condition-code steps (estimate, two Newton steps, quotient and one
+// correction).
+__device__ __forceinline__ double div64(double n, double d) {
+  double r = __builtin_amdgcn_rcp(d);
+  r = __builtin_fma(__builtin_fma(-d, r, 1.0), r, r);
+  r = __builtin_fma(__builtin_fma(-d, r, 1.0), r, r);
+  const double q = n * r;
+  return __builtin_fma(__builtin_fma(-d, q, n), r, q);
+}
+
+// n / d with r the correctly rounded 1 / d at hand: correctly rounded (Markstein
+// 1990) in three instructions.
+__device__ __forceinline__ double div64(double n, double d, double r) {
+  const double q = n * r;
+  return __builtin_fma(__builtin_fma(-d, q, n), r, q);
+}
+
 // One side of WENO-Z5 (Z) or WENO5-JS from five points, upwind first, in the
 // form above: the face value is f2 + the return value / 6.  eps4 = 4 eps.
 template <bool Z>
