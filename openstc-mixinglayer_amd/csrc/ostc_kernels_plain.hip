@@ -1,36 +1,59 @@
 // ostc_kernels_plain.hip -- per-block kernels launched the way the reference
-// launches them (src/RK.cuh:85-226): 64-thread pencils per direction for the
-// inviscid and viscous fluxes with dq read-modify-write in HBM, an (8,8,4)
-// interior grid for the update and local time step, a two-pass MIN with a
-// host read-back for dt, and one launch per boundary or inner face.  This is
+// launches them (src/RK.cuh:85-226): one kernel per direction for the inviscid
+// and viscous fluxes with dq read-modify-write in HBM, an (8,8,4) interior grid
+// for the update and local time step, a two-pass MIN with a host read-back for
+// dt, and one launch per boundary or inner face.  This is
 // the drop-in path; the fused batched kernel lives in ostc_kernels_fused.hip.
 #include "ostc_kernels.hpp"
 
 namespace ostc {
 
-// compute_convective_term_weno_{x,y,z} (src/WENO.cu:8-461): one 64-thread
-// block makes 64 face fluxes and updates 63 cells along DIR.  Launch grid
-// (segments along DIR, other axis a, other axis b).
+// A workgroup of the directional kernels makes F face fluxes of TW pencils
+// along DIR and updates F - 1 cells of each.  Along x the lanes run along the
+// pencil; along y and z the pencils are neighbours in i, so that 16 lanes read
+// one 128-byte line of a plane (a pencil a workgroup, as along x, reads 8 bytes
+// of each line: 96x80x64 cells, AUSM+ 104 / 133 us along y / z against 23 us
+// along x, viscous 155 / 226 against 27).
+template <int DIR>
+struct Pencil {
+  static constexpr int TW = DIR == 0 ? 1 : 16, F = DIR == 0 ? 64 : 16, T = TW * F;
+};
+
+// Cell index of position pos along DIR of pencil col, of workgroup
+// (segment, other axis a, other axis b), a in steps of TW.
+template <int DIR>
+__device__ __forceinline__ void pencil_idx(int pos, int col, int ijk[3]) {
+  const int a = Pencil<DIR>::TW * blockIdx.y + col, b = blockIdx.z;
+  ijk[0] = DIR == 0 ? pos : a;
+  ijk[1] = DIR == 0 ? a : (DIR == 1 ? pos : b);
+  ijk[2] = DIR == 2 ? pos : b;
+}
+template <int DIR>
+__device__ __forceinline__ bool pencil_inside(const DevBlock& B, int col) {
+  return Pencil<DIR>::TW * (int)blockIdx.y + col < (DIR == 0 ? B.my : B.mx);
+}
+
+// compute_convective_term_weno_{x,y,z} (src/WENO.cu:8-461): F face fluxes of
+// TW pencils and F - 1 updated cells of each.
 template <int DIR, int SCHEME>
-__global__ __launch_bounds__(64) void k_weno_pencil(DevBlock B, Params P, int slot) {
+__global__ __launch_bounds__(Pencil<DIR>::T) void k_weno_pencil(DevBlock B, Params P, int slot) {
   constexpr int R = Stencil<SCHEME>::R, W = Stencil<SCHEME>::W;
-  constexpr int NP = 63 + 2 * R;
-  __shared__ double sFp[5][NP], sFm[5][NP], sFc[5][64];
+  constexpr int TW = Pencil<DIR>::TW, F = Pencil<DIR>::F, T = Pencil<DIR>::T;
+  constexpr int NP = F - 1 + 2 * R;
+  __shared__ double sFp[5][NP * TW], sFm[5][NP * TW], sFc[5][T];
   const int m = DIR == 0 ? B.mx : (DIR == 1 ? B.my : B.mz);
-  const int c0 = 63 * blockIdx.x;
+  const int c0 = (F - 1) * blockIdx.x;
   const int tid = threadIdx.x;
-  int base[3];
-  if (DIR == 0) { base[1] = blockIdx.y; base[2] = blockIdx.z; }
-  if (DIR == 1) { base[0] = blockIdx.y; base[2] = blockIdx.z; }
-  if (DIR == 2) { base[0] = blockIdx.y; base[1] = blockIdx.z; }
+  const int col = tid % TW, f = tid / TW;
+  const bool inside = pencil_inside<DIR>(B, col);  // T is a multiple of TW: col stays over the strides
   const double* cv = B.cv[slot];
   const double* bv = B.bv[slot];
   const long long s = B.sz;
-  for (int pt = tid; pt < NP; pt += 64) {
-    const int pos = c0 - R + pt;
-    if (pos > m - 1 + R) continue;
-    int ijk[3] = {base[0], base[1], base[2]};
-    ijk[DIR] = pos;
+  for (int pt = tid; pt < NP * TW; pt += T) {
+    const int pos = c0 - R + pt / TW;
+    if (!inside || pos > m - 1 + R) continue;
+    int ijk[3];
+    pencil_idx<DIR>(pos, col, ijk);
     const long long p = pidx(B, ijk[0], ijk[1], ijk[2]);
     double q[5];
     for (int l = 0; l < 5; ++l) q[l] = cv[p + l * s];
@@ -41,15 +64,15 @@ __global__ __launch_bounds__(64) void k_weno_pencil(DevBlock B, Params P, int sl
     for (int l = 0; l < 5; ++l) { sFp[l][pt] = fp[l]; sFm[l][pt] = fm[l]; }
   }
   __syncthreads();
-  const int L = c0 - 1 + tid;  // face L+1/2
-  if (L <= m - 1) {
-    int ijk[3] = {base[0], base[1], base[2]};
-    ijk[DIR] = L;
+  const int L = c0 - 1 + f;  // face L+1/2
+  if (inside && L <= m - 1) {
+    int ijk[3];
+    pencil_idx<DIR>(L, col, ijk);
     const long long p1 = pidx(B, ijk[0], ijk[1], ijk[2]);
     ijk[DIR] = L + 1;
     const long long p2 = pidx(B, ijk[0], ijk[1], ijk[2]);
     const double j1 = B.jac[p1], j2 = B.jac[p2];
-    const int sL = tid + R - 1;  // LDS index of cell L
+    const int sL = tid + (R - 1) * TW;  // LDS index of cell L
     if constexpr (SCHEME == 52 || SCHEME == 72) {
       // compute_weno_flux_ch<Air>, "method 1" (src/WENO.cu:1147-1453): the
       // W split fluxes of each side projected on the left eigenvectors of
@@ -74,11 +97,11 @@ __global__ __launch_bounds__(64) void k_weno_pencil(DevBlock B, Params P, int sl
       for (int l = 0; l < 5; ++l) {
         double vp[W], vm[W];
         for (int r = 0; r < W; ++r) {
-          vp[r] = M.L[l][0] * sFp[0][sL - W / 2 + r];
-          vm[r] = M.L[l][0] * sFm[0][sL - W / 2 + 1 + r];
+          vp[r] = M.L[l][0] * sFp[0][sL + (r - W / 2) * TW];
+          vm[r] = M.L[l][0] * sFm[0][sL + (r - W / 2 + 1) * TW];
           for (int n = 1; n < 5; ++n) {
-            vp[r] += M.L[l][n] * sFp[n][sL - W / 2 + r];
-            vm[r] += M.L[l][n] * sFm[n][sL - W / 2 + 1 + r];
+            vp[r] += M.L[l][n] * sFp[n][sL + (r - W / 2) * TW];
+            vm[r] += M.L[l][n] * sFm[n][sL + (r - W / 2 + 1) * TW];
           }
         }
         if constexpr (SCHEME == 72) fChar[l] = weno7z(vp, vm, e);
@@ -97,8 +120,8 @@ __global__ __launch_bounds__(64) void k_weno_pencil(DevBlock B, Params P, int sl
     for (int l = 0; l < 5; ++l) {
       double vp[W], vm[W];
       for (int r = 0; r < W; ++r) {
-        vp[r] = sFp[l][sL - (W / 2) + r];
-        vm[r] = sFm[l][sL - (W / 2) + 1 + r];
+        vp[r] = sFp[l][sL + (r - W / 2) * TW];
+        vm[r] = sFm[l][sL + (r - W / 2 + 1) * TW];
       }
       const double e = l == 0 ? eps3[0] : (l == 4 ? eps3[2] : eps3[1]);
       sFc[l][tid] = weno_face<SCHEME>(vp, vm, e);
@@ -106,40 +129,41 @@ __global__ __launch_bounds__(64) void k_weno_pencil(DevBlock B, Params P, int sl
     }
   }
   __syncthreads();
-  if (tid > 0 && L <= m - 1) {
-    int ijk[3] = {base[0], base[1], base[2]};
-    ijk[DIR] = L;
+  if (f > 0 && inside && L <= m - 1) {
+    int ijk[3];
+    pencil_idx<DIR>(L, col, ijk);
     const long long p0 = pidx0(B, ijk[0], ijk[1], ijk[2]);
-    for (int l = 0; l < 5; ++l) B.dq[p0 + l * B.n0] -= sFc[l][tid] - sFc[l][tid - 1];
+    for (int l = 0; l < 5; ++l) B.dq[p0 + l * B.n0] -= sFc[l][tid] - sFc[l][tid - TW];
   }
 }
 
 // compute_convective_term_ep_1D<Air> (src/InviscidScheme.cu:550-768), the
 // sixth-order energy-preserving scheme (inviscid_scheme 6; Pirozzoli,
 // J. Comput. Phys. 230 (2011) 2997-3014): rho, u, v, w, p, H = (E + p)/rho,
-// the metric row, J and UJ = (k . u) J of 69 pencil points in LDS; the
-// two-point fluxes T(i, l), l = 1..3, of 66 points; 64 face fluxes
+// the metric row, J and UJ = (k . u) J of the pencils' points in LDS; the
+// two-point fluxes T(i, l), l = 1..3, of F + 2 points; F face fluxes
 // 2 (3/4 T(i,1) - 3/20 (T(i,2) + T(i-1,2)) + 1/60 (T(i,3) + T(i-1,3) +
-// T(i-2,3))); 63 cells updated.
+// T(i-2,3))); F - 1 cells updated.
 template <int DIR>
-__global__ __launch_bounds__(64) void k_ep_pencil(DevBlock B, int slot) {
-  constexpr int R = 3, NP = 63 + 2 * R, NT = 66;
-  __shared__ double sP[11][NP], sT[3][5][NT], sFc[5][64];
+__global__ __launch_bounds__(Pencil<DIR>::T) void k_ep_pencil(DevBlock B, int slot) {
+  constexpr int TW = Pencil<DIR>::TW, F = Pencil<DIR>::F, T = Pencil<DIR>::T;
+  constexpr int R = 3, NP = F - 1 + 2 * R, NT = F + 2;
+  __shared__ double sP[11][NP * TW], sT[3][5][NT * TW];
+  double(*sFc)[T] = reinterpret_cast<double(*)[T]>(&sP[0][0]);  // over the points once the T(i, l) are formed
+  static_assert(5 * T <= 11 * NP * TW);
   const int m = DIR == 0 ? B.mx : (DIR == 1 ? B.my : B.mz);
-  const int c0 = 63 * blockIdx.x;
+  const int c0 = (F - 1) * blockIdx.x;
   const int tid = threadIdx.x;
-  int base[3];
-  if (DIR == 0) { base[1] = blockIdx.y; base[2] = blockIdx.z; }
-  if (DIR == 1) { base[0] = blockIdx.y; base[2] = blockIdx.z; }
-  if (DIR == 2) { base[0] = blockIdx.y; base[1] = blockIdx.z; }
+  const int col = tid % TW, f = tid / TW;
+  const bool inside = pencil_inside<DIR>(B, col);  // T is a multiple of TW: col stays over the strides
   const double* cv = B.cv[slot];
   const double* bv = B.bv[slot];
   const long long s = B.sz;
-  for (int pt = tid; pt < NP; pt += 64) {
-    const int pos = c0 - R + pt;
-    if (pos > m - 1 + R) continue;
-    int ijk[3] = {base[0], base[1], base[2]};
-    ijk[DIR] = pos;
+  for (int pt = tid; pt < NP * TW; pt += T) {
+    const int pos = c0 - R + pt / TW;
+    if (!inside || pos > m - 1 + R) continue;
+    int ijk[3];
+    pencil_idx<DIR>(pos, col, ijk);
     const long long p = pidx(B, ijk[0], ijk[1], ijk[2]);
 #pragma unroll
     for (int l = 0; l < 5; ++l) sP[l][pt] = bv[p + l * s];
@@ -155,12 +179,12 @@ __global__ __launch_bounds__(64) void k_ep_pencil(DevBlock B, int slot) {
     sP[10][pt] = uk;
   }
   __syncthreads();
-  for (int t = tid; t < NT; t += 64) {
-    const int pos = c0 - R + t;
+  for (int t = tid; t < NT * TW; t += T) {
+    const int pos = c0 - R + t / TW;
 #pragma unroll
     for (int l = 1; l <= 3; ++l) {
-      if (pos + l > m - 1 + R) continue;
-      const int a = t, b = t + l;
+      if (!inside || pos + l > m - 1 + R) continue;
+      const int a = t, b = t + l * TW;
       const double weight = 0.125 * (sP[10][a] + sP[10][b]) * (sP[0][a] + sP[0][b]);
       const double pWeight = 0.25 * (sP[4][a] + sP[4][b]);
       sT[l - 1][0][t] = 2 * weight;
@@ -171,46 +195,45 @@ __global__ __launch_bounds__(64) void k_ep_pencil(DevBlock B, int slot) {
     }
   }
   __syncthreads();
-  const int L = c0 - 1 + tid;  // face L+1/2
-  if (L <= m - 1) {
+  const int L = c0 - 1 + f;  // face L+1/2
+  if (inside && L <= m - 1) {
     constexpr double central_1[3] = {0.75, -3.0 / 20, 1.0 / 60};
-    const int t = tid + R - 1;  // point L
+    const int t = tid + (R - 1) * TW;  // point L
 #pragma unroll
     for (int l = 0; l < 5; ++l)
-      sFc[l][tid] = 2 * (central_1[0] * sT[0][l][t] + central_1[1] * (sT[1][l][t] + sT[1][l][t - 1]) +
-                         central_1[2] * (sT[2][l][t] + sT[2][l][t - 1] + sT[2][l][t - 2]));
+      sFc[l][tid] = 2 * (central_1[0] * sT[0][l][t] + central_1[1] * (sT[1][l][t] + sT[1][l][t - TW]) +
+                         central_1[2] * (sT[2][l][t] + sT[2][l][t - TW] + sT[2][l][t - 2 * TW]));
   }
   __syncthreads();
-  if (tid > 0 && L <= m - 1) {
-    int ijk[3] = {base[0], base[1], base[2]};
-    ijk[DIR] = L;
+  if (f > 0 && inside && L <= m - 1) {
+    int ijk[3];
+    pencil_idx<DIR>(L, col, ijk);
     const long long p0 = pidx0(B, ijk[0], ijk[1], ijk[2]);
-    for (int l = 0; l < 5; ++l) B.dq[p0 + l * B.n0] -= sFc[l][tid] - sFc[l][tid - 1];
+    for (int l = 0; l < 5; ++l) B.dq[p0 + l * B.n0] -= sFc[l][tid] - sFc[l][tid - TW];
   }
 }
 
 // compute_convective_term_pv_1D<Air> (src/InviscidScheme.cu:50-165): the
-// primitive variables of 67 pencil points staged in LDS, MUSCL / NND2 /
+// primitive variables of the pencils' points staged in LDS, MUSCL / NND2 /
 // first-order reconstruction (src/Reconstruction.cu:5-46) and an LF, AUSM+ or
-// HLLC flux (src/RiemannSolver.cuh) at 64 faces, 63 cells updated.
+// HLLC flux (src/RiemannSolver.cuh) at F faces, F - 1 cells updated.
 template <int DIR>
-__global__ __launch_bounds__(64) void k_pv_pencil(DevBlock B, Params P, int slot) {
-  constexpr int NP = 67;  // points c0-2 .. c0+64
-  __shared__ double sPv[5][NP], sK[3][NP], sJ[NP], sFc[5][64], sDelta[NP];
+__global__ __launch_bounds__(Pencil<DIR>::T) void k_pv_pencil(DevBlock B, Params P, int slot) {
+  constexpr int TW = Pencil<DIR>::TW, F = Pencil<DIR>::F, T = Pencil<DIR>::T;
+  constexpr int NP = F + 3;  // points c0-2 .. c0+F
+  __shared__ double sPv[5][NP * TW], sK[3][NP * TW], sJ[NP * TW], sFc[5][T], sDelta[NP * TW];
   const int m = DIR == 0 ? B.mx : (DIR == 1 ? B.my : B.mz);
-  const int c0 = 63 * blockIdx.x;
+  const int c0 = (F - 1) * blockIdx.x;
   const int tid = threadIdx.x;
-  int base[3];
-  if (DIR == 0) { base[1] = blockIdx.y; base[2] = blockIdx.z; }
-  if (DIR == 1) { base[0] = blockIdx.y; base[2] = blockIdx.z; }
-  if (DIR == 2) { base[0] = blockIdx.y; base[1] = blockIdx.z; }
+  const int col = tid % TW, f = tid / TW;
+  const bool inside = pencil_inside<DIR>(B, col);  // T is a multiple of TW: col stays over the strides
   const double* bv = B.bv[slot];
   const long long s = B.sz;
-  for (int pt = tid; pt < NP; pt += 64) {
-    const int pos = c0 - 2 + pt;
-    if (pos > m + 1) continue;  // the faces need points -2 .. m+1 (ngg >= 2)
-    int ijk[3] = {base[0], base[1], base[2]};
-    ijk[DIR] = pos;
+  for (int pt = tid; pt < NP * TW; pt += T) {
+    const int pos = c0 - 2 + pt / TW;
+    if (!inside || pos > m + 1) continue;  // the faces need points -2 .. m+1 (ngg >= 2)
+    int ijk[3];
+    pencil_idx<DIR>(pos, col, ijk);
     const long long p = pidx(B, ijk[0], ijk[1], ijk[2]);
     for (int l = 0; l < 5; ++l) sPv[l][pt] = bv[p + l * s];
     for (int c = 0; c < 3; ++c) sK[c][pt] = B.met[p + (3 * DIR + c) * s];
@@ -223,32 +246,32 @@ __global__ __launch_bounds__(64) void k_pv_pencil(DevBlock B, Params P, int slot
     }
   }
   __syncthreads();
-  const int L = c0 - 1 + tid;  // face L+1/2 between LDS points tid+1 and tid+2
-  if (L <= m - 1) {
+  const int L = c0 - 1 + f, p1 = tid + TW, p2 = tid + 2 * TW;  // face L+1/2 between LDS points p1 and p2
+  if (inside && L <= m - 1) {
     double pl[6], pr[6];
     for (int l = 0; l < 5; ++l)
-      reconstruct_var(P.recon, sPv[l][tid], sPv[l][tid + 1], sPv[l][tid + 2], sPv[l][tid + 3], &pl[l], &pr[l]);
+      reconstruct_var(P.recon, sPv[l][tid], sPv[l][p1], sPv[l][p2], sPv[l][p2 + TW], &pl[l], &pr[l]);
     // total energy of the reconstructed states, reconstruction<Air> (src/InviscidScheme.cu:210-215)
     const double el = 0.5 * (pl[1] * pl[1] + pl[2] * pl[2] + pl[3] * pl[3]);
     const double er = 0.5 * (pr[1] * pr[1] + pr[2] * pr[2] + pr[3] * pr[3]);
     pl[5] = el * pl[0] + pl[4] / (kGamma - 1);
     pr[5] = er * pr[0] + pr[4] / (kGamma - 1);
-    const double ml[3] = {sK[0][tid + 1], sK[1][tid + 1], sK[2][tid + 1]};
-    const double mr[3] = {sK[0][tid + 2], sK[1][tid + 2], sK[2][tid + 2]};
-    double f[5];
+    const double ml[3] = {sK[0][p1], sK[1][p1], sK[2][p1]};
+    const double mr[3] = {sK[0][p2], sK[1][p2], sK[2][p2]};
+    double fl[5];
     if (P.scheme == 2) {
-      roe_air(pl, pr, ml, mr, sJ[tid + 1], sJ[tid + 2], sDelta[tid + 1], sDelta[tid + 2], f);
+      roe_air(pl, pr, ml, mr, sJ[p1], sJ[p2], sDelta[p1], sDelta[p2], fl);
     } else {
-      riemann_air(P.scheme, pl, pr, ml, mr, sJ[tid + 1], sJ[tid + 2], f);
+      riemann_air(P.scheme, pl, pr, ml, mr, sJ[p1], sJ[p2], fl);
     }
-    for (int l = 0; l < 5; ++l) sFc[l][tid] = f[l];
+    for (int l = 0; l < 5; ++l) sFc[l][tid] = fl[l];
   }
   __syncthreads();
-  if (tid > 0 && L <= m - 1) {
-    int ijk[3] = {base[0], base[1], base[2]};
-    ijk[DIR] = L;
+  if (f > 0 && inside && L <= m - 1) {
+    int ijk[3];
+    pencil_idx<DIR>(L, col, ijk);
     const long long p0 = pidx0(B, ijk[0], ijk[1], ijk[2]);
-    for (int l = 0; l < 5; ++l) B.dq[p0 + l * B.n0] -= sFc[l][tid] - sFc[l][tid - 1];
+    for (int l = 0; l < 5; ++l) B.dq[p0 + l * B.n0] -= sFc[l][tid] - sFc[l][tid - TW];
   }
 }
 
@@ -278,20 +301,19 @@ __device__ __forceinline__ void face_gradients(PV pv, int i, int j, int k, doubl
 
 // viscous_flux_{fv,gv,hv} (src/SchemeSelector.cuh:69-154).
 template <int DIR>
-__global__ __launch_bounds__(64) void k_visc_pencil(DevBlock B, Params P, int slot) {
-  __shared__ double sFv[4][64];
+__global__ __launch_bounds__(Pencil<DIR>::T) void k_visc_pencil(DevBlock B, Params P, int slot) {
+  constexpr int TW = Pencil<DIR>::TW, F = Pencil<DIR>::F, T = Pencil<DIR>::T;
+  __shared__ double sFv[4][T];
   const int m = DIR == 0 ? B.mx : (DIR == 1 ? B.my : B.mz);
-  const int tid = threadIdx.x;
-  const int L = 63 * blockIdx.x - 1 + tid;
+  const int tid = threadIdx.x, col = tid % TW, f = tid / TW;
+  const int L = (F - 1) * blockIdx.x - 1 + f;
   int ijk[3];
-  if (DIR == 0) { ijk[1] = blockIdx.y; ijk[2] = blockIdx.z; }
-  if (DIR == 1) { ijk[0] = blockIdx.y; ijk[2] = blockIdx.z; }
-  if (DIR == 2) { ijk[0] = blockIdx.y; ijk[1] = blockIdx.z; }
-  ijk[DIR] = L;
+  pencil_idx<DIR>(L, col, ijk);
+  const bool active = pencil_inside<DIR>(B, col) && L <= m - 1;
   const double* bv = B.bv[slot];
   const double* mu = B.mul[slot];
   const long long s = B.sz;
-  if (L <= m - 1) {
+  if (active) {
     auto pv = [&](int a, int b, int c, int l) { return bv[pidx(B, a, b, c) + l * s]; };
     double d[4][3];
     face_gradients<DIR>(pv, ijk[0], ijk[1], ijk[2], d);
@@ -309,9 +331,9 @@ __global__ __launch_bounds__(64) void k_visc_pencil(DevBlock B, Params P, int sl
     for (int l = 0; l < 4; ++l) sFv[l][tid] = fv[l];
   }
   __syncthreads();
-  if (tid > 0 && L <= m - 1) {
+  if (f > 0 && active) {
     const long long p0 = pidx0(B, ijk[0], ijk[1], ijk[2]);
-    for (int l = 0; l < 4; ++l) B.dq[p0 + (l + 1) * B.n0] += sFv[l][tid] - sFv[l][tid - 1];
+    for (int l = 0; l < 4; ++l) B.dq[p0 + (l + 1) * B.n0] += sFv[l][tid] - sFv[l][tid - TW];
   }
 }
 
@@ -492,17 +514,17 @@ __global__ __launch_bounds__(256) void k_residual(DevBlock B, double* out4) {
 // ------------------------------------------------------------- launchers
 static dim3 pencil_grid(const DevBlock& B, int dir) {
   const int m = dir == 0 ? B.mx : (dir == 1 ? B.my : B.mz);
-  const unsigned seg = (m - 1) / 63 + 1;
+  const int cells = dir == 0 ? Pencil<0>::F - 1 : Pencil<1>::F - 1, tw = Pencil<1>::TW;
+  const unsigned seg = (m - 1) / cells + 1;
   if (dir == 0) return dim3(seg, B.my, B.mz);
-  if (dir == 1) return dim3(seg, B.mx, B.mz);
-  return dim3(seg, B.mx, B.my);
+  return dim3(seg, (B.mx - 1) / tw + 1, dir == 1 ? B.mz : B.my);
 }
 
 template <int SCHEME>
 static void launch_weno(const DevBlock& B, const Params& P, hipStream_t st, long long* n) {
-  hipLaunchKernelGGL((k_weno_pencil<0, SCHEME>), pencil_grid(B, 0), dim3(64), 0, st, B, P, 0);
-  hipLaunchKernelGGL((k_weno_pencil<1, SCHEME>), pencil_grid(B, 1), dim3(64), 0, st, B, P, 0);
-  hipLaunchKernelGGL((k_weno_pencil<2, SCHEME>), pencil_grid(B, 2), dim3(64), 0, st, B, P, 0);
+  hipLaunchKernelGGL((k_weno_pencil<0, SCHEME>), pencil_grid(B, 0), dim3(Pencil<0>::T), 0, st, B, P, 0);
+  hipLaunchKernelGGL((k_weno_pencil<1, SCHEME>), pencil_grid(B, 1), dim3(Pencil<1>::T), 0, st, B, P, 0);
+  hipLaunchKernelGGL((k_weno_pencil<2, SCHEME>), pencil_grid(B, 2), dim3(Pencil<2>::T), 0, st, B, P, 0);
   *n += 3;
 }
 
@@ -546,21 +568,21 @@ void plain_rhs(const DevBlock& B, const Params& P, hipStream_t st, long long* n)
   else if (P.scheme == 52) launch_weno<52>(B, P, st, n);
   else if (P.scheme == 72) launch_weno<72>(B, P, st, n);
   else if (P.scheme == 6) {
-    hipLaunchKernelGGL(k_ep_pencil<0>, pencil_grid(B, 0), dim3(64), 0, st, B, 0);
-    hipLaunchKernelGGL(k_ep_pencil<1>, pencil_grid(B, 1), dim3(64), 0, st, B, 0);
-    hipLaunchKernelGGL(k_ep_pencil<2>, pencil_grid(B, 2), dim3(64), 0, st, B, 0);
+    hipLaunchKernelGGL(k_ep_pencil<0>, pencil_grid(B, 0), dim3(Pencil<0>::T), 0, st, B, 0);
+    hipLaunchKernelGGL(k_ep_pencil<1>, pencil_grid(B, 1), dim3(Pencil<1>::T), 0, st, B, 0);
+    hipLaunchKernelGGL(k_ep_pencil<2>, pencil_grid(B, 2), dim3(Pencil<2>::T), 0, st, B, 0);
     *n += 3;
   }
   else if (P.scheme == 1 || P.scheme == 2 || P.scheme == 3 || P.scheme == 4) {
-    hipLaunchKernelGGL(k_pv_pencil<0>, pencil_grid(B, 0), dim3(64), 0, st, B, P, 0);
-    hipLaunchKernelGGL(k_pv_pencil<1>, pencil_grid(B, 1), dim3(64), 0, st, B, P, 0);
-    hipLaunchKernelGGL(k_pv_pencil<2>, pencil_grid(B, 2), dim3(64), 0, st, B, P, 0);
+    hipLaunchKernelGGL(k_pv_pencil<0>, pencil_grid(B, 0), dim3(Pencil<0>::T), 0, st, B, P, 0);
+    hipLaunchKernelGGL(k_pv_pencil<1>, pencil_grid(B, 1), dim3(Pencil<1>::T), 0, st, B, P, 0);
+    hipLaunchKernelGGL(k_pv_pencil<2>, pencil_grid(B, 2), dim3(Pencil<2>::T), 0, st, B, P, 0);
     *n += 3;
   } else launch_weno<51>(B, P, st, n);
   if (P.visc) {
-    hipLaunchKernelGGL(k_visc_pencil<0>, pencil_grid(B, 0), dim3(64), 0, st, B, P, 0);
-    hipLaunchKernelGGL(k_visc_pencil<1>, pencil_grid(B, 1), dim3(64), 0, st, B, P, 0);
-    hipLaunchKernelGGL(k_visc_pencil<2>, pencil_grid(B, 2), dim3(64), 0, st, B, P, 0);
+    hipLaunchKernelGGL(k_visc_pencil<0>, pencil_grid(B, 0), dim3(Pencil<0>::T), 0, st, B, P, 0);
+    hipLaunchKernelGGL(k_visc_pencil<1>, pencil_grid(B, 1), dim3(Pencil<1>::T), 0, st, B, P, 0);
+    hipLaunchKernelGGL(k_visc_pencil<2>, pencil_grid(B, 2), dim3(Pencil<2>::T), 0, st, B, P, 0);
     *n += 3;
   }
 }
