@@ -64,7 +64,7 @@ struct HBlock {
   DevBlock d{};
 };
 
-struct Group { int lo = 0, hi = 0; long long total = 0; };
+struct Group { int lo = 0, hi = 0, wg_lo = 0, n_wg = 0; bool face_state = false; };  // ops lo..hi-1, one launch
 
 struct Access { int block; Box box; };
 
@@ -101,10 +101,12 @@ struct ostc_ctx_s {
   DevBlock* d_blocks = nullptr;
   std::vector<DevOp> ops;
   DevOp* d_ops = nullptr;
+  OpWg* d_op_wg = nullptr;
   std::vector<Group> bc_rounds, comm_levels;
   Group props, rim;
-  std::vector<std::vector<int>> plain_bc;
-  std::vector<int> plain_comm;
+  std::vector<std::vector<Group>> plain_bc;  // one block's boundary ops
+  std::vector<std::vector<int>> bc_order;    // the same ops in the reference's order
+  std::vector<Group> plain_comm;             // one inner face each, in the reference's order
   int tile_index = 0, n_wg = 0, xcd_remap = 1, n_tiles = 0, waves = 0, split = 0;
   int* d_tile_block = nullptr;
   SweepPlan sweep{};       // work lists of the inviscid sweeps (component-wise WENO schemes)
@@ -190,6 +192,7 @@ DevOp make_op(int type, int block, const Box& b) {
     op.n[d] = b.hi[d] - b.lo[d] + 1;
   }
   op.count = (long long)op.n[0] * op.n[1] * op.n[2];
+  op.layers = 1;
   return op;
 }
 
@@ -226,16 +229,36 @@ Box box_and(const Box& a, const Box& b) {
   return r;
 }
 
-// Work-lists for the ghost layers.  Boundary ops of one block keep the
-// reference's sequential order (one launch "round" per position in the
-// block's priority-sorted list; blocks are independent).  Inner-face ops keep
-// the reference's order (blocks, then faces) only between ops whose cell
-// sets conflict: each op gets level 1 + the highest level of an earlier
-// conflicting op, and one launch runs one level.
+// An op with the boxes it writes and reads, and its launch: 1 + the last launch
+// of an earlier op that it conflicts with.
+struct LeveledOp { DevOp op; std::vector<Access> w, r; int level; };
+
+bool meet(const std::vector<Access>& x, const std::vector<Access>& y) {
+  for (auto& u : x)
+    for (auto& v : y)
+      if (u.block == v.block && box_hit(u.box, v.box)) return true;
+  return false;
+}
+
+// the level of o after the first n ops of a list
+int level_after(const std::vector<LeveledOp>& ops, size_t n, const LeveledOp& o) {
+  int level = 0;
+  for (size_t q = 0; q < n; ++q) {
+    const LeveledOp& e = ops[q];
+    if (e.level >= level && (meet(e.w, o.w) || meet(e.w, o.r) || meet(e.r, o.w))) level = e.level + 1;
+  }
+  return level;
+}
+
+// Work-lists for the ghost layers.  Ops keep the reference's order (a block's
+// boundary faces by priority; inner faces by block and face) only between ops
+// whose cell sets conflict (LeveledOp), and one launch runs one level of all
+// blocks: two opposite faces of a block, which the reference takes one after
+// the other, share a launch.
 int build_ops(ostc_ctx c) {
   const int G = c->ngg;
   const int nb = (int)c->blocks.size();
-  std::vector<std::vector<DevOp>> bc_of_block(nb);
+  std::vector<std::vector<LeveledOp>> bc_of_block(nb);
   std::vector<DevOp> rim_ops, props_ops;
   for (int b = 0; b < nb; ++b) {
     HBlock& B = c->blocks[b];
@@ -258,11 +281,17 @@ int build_ops(ostc_ctx c) {
         op.aux = c->d_inflow + fd.y_off;
         op.pass = c->d_pass;
       }
-      bc_of_block[b].push_back(op);
+      const bool copies = ot == OP_BC_OUTFLOW || ot == OP_BC_PERIODIC;
+      if (copies) op.layers = G;
       // ghost cells this op reads before the same stage can have written them
       Box rd = fd.type == OSTC_BC_PERIODIC
                    ? (fd.r.side < 0 ? face_box(fd.r, m - 1 - G, m - 2) : face_box(fd.r, 1, G))
                    : face_box(fd.r, idx, idx);
+      // written: the ghost layers, with a far-field or inflow state the face too
+      const int off = copies ? 1 : 0;
+      LeveledOp o{op, {{b, fd.r.side < 0 ? face_box(fd.r, -G, -off) : face_box(fd.r, idx + off, idx + G)}}, {{b, rd}}, 0};
+      o.level = level_after(bc_of_block[b], bc_of_block[b].size(), o);
+      bc_of_block[b].push_back(o);
       for (const Box& rb : minus_interior(rd, B.m)) rim_ops.push_back(make_op(OP_COPY_BV, b, rb));
       if (fd.type == OSTC_BC_FARFIELD || fd.type == OSTC_BC_INFLOW) {
         // the boundary state replaces the face points after the fused update
@@ -284,7 +313,7 @@ int build_ops(ostc_ctx c) {
   // face of a two-sided interface into
   //  * a bulk part, the face without a frame of ngg+1 cells along its
   //    tangential rims: no other face's op reads or writes these cells, so
-  //    all bulk parts run in one launch; one side of the pair (the high face
+  //    all bulk parts run in the first launch; one side of the pair (the high face
   //    of a low/high pair, else the face registered first) averages the
   //    shared node layer and recomputes cv in both blocks, the other side
   //    copies its ghost layers only;
@@ -335,9 +364,17 @@ int build_ops(ostc_ctx c) {
     }
     return op;
   };
-  std::vector<DevOp> plain_ops, bulk_ops;
-  struct CommOp { DevOp op; std::vector<Access> w, r; int level; };
-  std::vector<CommOp> edge;
+  std::vector<DevOp> plain_ops;
+  std::vector<LeveledOp> bulk, edge;
+  auto leveled = [&](const FaceGeom& F, const Box& bx) {
+    LeveledOp o{comm_op(F, bx), {{F.A, bx}}, {{F.T, map_box(F.M, bx)}}, 0};
+    const Box sh = box_and(F.shA, bx);
+    if (box_ok(sh)) {
+      o.w.push_back({F.T, map_box(F.M, sh)});
+      o.r.push_back({F.A, sh});
+    }
+    return o;
+  };
   for (size_t q = 0; q < geo.size(); ++q) {
     const FaceGeom& F = geo[q];
     plain_ops.push_back(comm_op(F, F.box));
@@ -354,9 +391,8 @@ int build_ops(ostc_ctx c) {
         if (F.M.side < 0) cb.hi[a] = F.M.shared - 1;
         else cb.lo[a] = F.M.shared + 1;
       }
-      DevOp op = comm_op(F, cb);
-      if (averages) op.flags = 1;  // recompute the target block's cv on the shared layer
-      bulk_ops.push_back(op);
+      bulk.push_back(leveled(F, cb));
+      if (averages) bulk.back().op.flags = 1;  // recompute the target block's cv on the shared layer
       // frame = box minus core, as slabs along the first tangential axis
       // and then the second
       const int t1 = a == 0 ? 1 : 0, t2 = a == 2 ? 1 : 2;
@@ -369,90 +405,77 @@ int build_ops(ostc_ctx c) {
     } else {
       frame.push_back(F.box);
     }
-    for (const Box& eb : frame) {
-      CommOp co;
-      co.op = comm_op(F, eb);
-      const Box sh = box_and(F.shA, eb);
-      co.w = {{F.A, eb}, {F.T, map_box(F.M, sh)}};
-      co.r = {{F.T, map_box(F.M, eb)}, {F.A, sh}};
-      co.level = 0;
-      for (auto& e : edge) {
-        auto meet = [](const std::vector<Access>& x, const std::vector<Access>& y) {
-          for (auto& u : x)
-            for (auto& v : y)
-              if (u.block == v.block && box_hit(u.box, v.box)) return true;
-          return false;
-        };
-        if (meet(e.w, co.w) || meet(e.w, co.r) || meet(e.r, co.w)) co.level = std::max(co.level, e.level + 1);
-      }
-      edge.push_back(co);
-    }
+    for (const Box& eb : frame) edge.push_back(leveled(F, eb));
   }
+  // a frame op waits only for a bulk part that it meets: none, unless a face
+  // without a partner lies across one
+  for (size_t q = 0; q < edge.size(); ++q)
+    edge[q].level = std::max(level_after(edge, q, edge[q]), level_after(bulk, bulk.size(), edge[q]));
   // assemble: [bc rounds][comm levels][props][rim]
   c->ops.clear();
   c->bc_rounds.clear();
   c->comm_levels.clear();
-  c->plain_bc.assign(nb, {});
-  size_t rounds = 0;
-  for (auto& v : bc_of_block) rounds = std::max(rounds, v.size());
-  auto close_group = [&](Group& g, int lo) {
-    g.lo = lo;
-    g.hi = (int)c->ops.size();
-    long long acc = 0;
-    for (int i = g.lo; i < g.hi; ++i) { c->ops[i].begin = acc; acc += c->ops[i].count; }
-    g.total = acc;
-  };
-  for (size_t r = 0; r < rounds; ++r) {
-    const int lo = (int)c->ops.size();
-    for (int b = 0; b < nb; ++b)
-      if (r < bc_of_block[b].size()) {
-        c->plain_bc[b].push_back((int)c->ops.size());
-        c->ops.push_back(bc_of_block[b][r]);
-      }
-    Group g;
-    close_group(g, lo);
-    c->bc_rounds.push_back(g);
-  }
-  if (!bulk_ops.empty()) {
-    const int lo = (int)c->ops.size();
-    for (auto& o : bulk_ops) c->ops.push_back(o);
-    Group g;
-    close_group(g, lo);
-    c->comm_levels.push_back(g);
-  }
-  int max_level = -1;
-  for (auto& e : edge) max_level = std::max(max_level, e.level);
-  for (int L = 0; L <= max_level; ++L) {
-    const int lo = (int)c->ops.size();
-    for (size_t q = 0; q < edge.size(); ++q)
-      if (edge[q].level == L) c->ops.push_back(edge[q].op);
-    Group g;
-    close_group(g, lo);
-    c->comm_levels.push_back(g);
-  }
   c->plain_comm.clear();
-  for (auto& o : plain_ops) {
-    // one launch per face: each op is a group of its own (begin = 0)
-    c->plain_comm.push_back((int)c->ops.size());
-    o.begin = 0;
+  c->plain_bc.assign(nb, {});
+  c->bc_order.assign(nb, {});
+  std::vector<OpWg> wgs;
+  // one launch of the ops added by f
+  auto group = [&](auto f) {
+    Group g;
+    g.lo = (int)c->ops.size();
+    g.wg_lo = (int)wgs.size();
+    f();
+    g.hi = (int)c->ops.size();
+    g.n_wg = (int)wgs.size() - g.wg_lo;
+    for (int q = g.lo; q < g.hi; ++q)
+      g.face_state = g.face_state || c->ops[q].type == OP_BC_FARFIELD || c->ops[q].type == OP_BC_INFLOW;
+    return g;
+  };
+  auto add = [&](const DevOp& o) {
+    for (long long first = 0; first < o.count * o.layers; first += kOpWg)
+      wgs.push_back(OpWg{(int)c->ops.size(), (int)first});
     c->ops.push_back(o);
+  };
+  int levels = 0;
+  for (int b = 0; b < nb; ++b) {
+    c->bc_order[b].resize(bc_of_block[b].size());
+    for (auto& o : bc_of_block[b]) levels = std::max(levels, o.level + 1);
   }
-  {
-    const int lo = (int)c->ops.size();
-    for (auto& o : props_ops) c->ops.push_back(o);
-    close_group(c->props, lo);
-  }
-  {
-    const int lo = (int)c->ops.size();
-    for (auto& o : rim_ops) c->ops.push_back(o);
-    close_group(c->rim, lo);
-  }
+  for (int L = 0; L < levels; ++L)
+    c->bc_rounds.push_back(group([&] {
+      for (int b = 0; b < nb; ++b) {
+        const Group g = group([&] {
+          for (size_t q = 0; q < bc_of_block[b].size(); ++q)
+            if (bc_of_block[b][q].level == L) {
+              c->bc_order[b][q] = (int)c->ops.size();
+              add(bc_of_block[b][q].op);
+            }
+        });
+        if (g.hi > g.lo) c->plain_bc[b].push_back(g);
+      }
+    }));
+  levels = bulk.empty() ? 0 : 1;
+  for (auto& e : edge) levels = std::max(levels, e.level + 1);
+  for (int L = 0; L < levels; ++L)
+    c->comm_levels.push_back(group([&] {
+      if (L == 0)
+        for (auto& o : bulk) add(o.op);
+      for (auto& o : edge)
+        if (o.level == L) add(o.op);
+    }));
+  for (auto& o : plain_ops) c->plain_comm.push_back(group([&] { add(o); }));
+  c->props = group([&] { for (auto& o : props_ops) add(o); });
+  c->rim = group([&] { for (auto& o : rim_ops) add(o); });
   if (!c->ops.empty()) {
     void* v = nullptr;
     HIPCHK(c, hipMalloc(&v, c->ops.size() * sizeof(DevOp)));
     c->allocs.push_back(v);
     c->d_ops = static_cast<DevOp*>(v);
     HIPCHK(c, hipMemcpy(c->d_ops, c->ops.data(), c->ops.size() * sizeof(DevOp), hipMemcpyHostToDevice));
+    HIPCHK(c, hipMalloc(&v, wgs.size() * sizeof(OpWg)));
+    c->allocs.push_back(v);
+    c->d_op_wg = static_cast<OpWg*>(v);
+    HIPCHK(c, hipMemcpy(c->d_op_wg, wgs.data(), wgs.size() * sizeof(OpWg), hipMemcpyHostToDevice));
   }
   return OSTC_OK;
 }
@@ -595,23 +618,18 @@ bool launch_stage(ostc_ctx c, int mode, const FusedArgs& a, long long* n) {
 }
 
 void launch_group(ostc_ctx c, const Group& g, int slot, int src, long long* n, bool props = false) {
-  if (g.hi > g.lo)
-    ops_launch(c->d_blocks, (int)c->blocks.size(), c->d_ops, g.lo, g.hi, g.total, slot, src, c->st, n, props);
-}
-
-void launch_op(ostc_ctx c, int idx, int slot, long long* n) {
-  ops_launch(c->d_blocks, (int)c->blocks.size(), c->d_ops, idx, idx + 1, c->ops[idx].count, slot, slot, c->st, n);
+  ops_launch(c->d_blocks, c->d_ops, c->d_op_wg + g.wg_lo, g.n_wg, g.face_state, slot, src, props, c->st, n);
 }
 
 // ---------------------------------------------------- per-block path pieces
 int plain_bc(ostc_ctx c, int b, long long* n) {
-  for (int idx : c->plain_bc[b]) launch_op(c, idx, 0, n);
+  for (const Group& g : c->plain_bc[b]) launch_group(c, g, 0, 0, n);
   if (c->inflow_noise) count_pass(c->d_pass, b, b + 1, c->st, n);
   return OSTC_OK;
 }
 
 int plain_exchange(ostc_ctx c, long long* n) {
-  for (int idx : c->plain_comm) launch_op(c, idx, 0, n);
+  for (const Group& g : c->plain_comm) launch_group(c, g, 0, 0, n);
   return OSTC_OK;
 }
 
@@ -1769,7 +1787,7 @@ int restore_state(ostc_ctx c, const DevBlock& B, const double* from) {
 // Transposed boundary copies of block b, in the reverse of their order.
 void bc_transpose(ostc_ctx c, int b, double* lam) {
   const DevBlock& B = c->blocks[b].d;
-  for (auto it = c->plain_bc[b].rbegin(); it != c->plain_bc[b].rend(); ++it) adj_bc_op(B, c->ops[*it], lam, c->st);
+  for (auto it = c->bc_order[b].rbegin(); it != c->bc_order[b].rend(); ++it) adj_bc_op(B, c->ops[*it], lam, c->st);
 }
 
 }  // namespace

@@ -14,8 +14,9 @@ void min_reduce(const double* in, long long len, double* scratch, int n_first, h
 void padded_pass(const DevBlock& B, int slot, int what, hipStream_t st, long long* n);
 void count_pass(unsigned long long* pass, int lo, int hi, hipStream_t st, long long* n);
 void sponge_mean(const DevBlock& B, const unsigned long long* iter, hipStream_t st, long long* n);
-void ops_launch(const DevBlock* d_blocks, int n_blocks, const DevOp* d_ops, int op_lo, int op_hi, long long total, int slot,
-                int src, hipStream_t st, long long* n, bool props = false);
+// n_wg workgroups of a launch; face_state: far-field or inflow ops among them
+void ops_launch(const DevBlock* blocks, const DevOp* ops, const OpWg* wgs, int n_wg, bool face_state, int slot, int src,
+                bool props, hipStream_t st, long long* n);
 // parallel faces (ring slot 0): pack into / unpack from buf + f.offset
 void par_pack(const DevBlock& B, const ParFace& f, double* buf, hipStream_t st);
 void par_unpack(const DevBlock& B, const ParFace& f, const double* recv, const double* sent, hipStream_t st);

@@ -426,49 +426,22 @@ __global__ __launch_bounds__(256) void k_padded(DevBlock B, int slot, int what) 
   const int j = blockIdx.y * blockDim.y + threadIdx.y - B.g;
   const int k = blockIdx.z * blockDim.z + threadIdx.z - B.g;
   if (i >= B.mx + B.g || j >= B.my + B.g || k >= B.mz + B.g) return;
-  DevOp op{};
-  op.type = what;
-  op.block = 0;
-  op.lo[0] = i; op.lo[1] = j; op.lo[2] = k;
-  op.n[0] = op.n[1] = op.n[2] = 1;
-  op_point(&B, op, 0, slot, slot);
+  const NodeArrays N = node_arrays(B, slot);
+  const long long p = pidx(B, i, j, k);
+  if (what == OP_PROPS) put_props(N, p, get_node(N, p));
+  else put_cv(N, p, get_node(N, p));
 }
 
-// One launch of a range of independent ops.  Thread -> op by binary search
-// over the ops' running point offsets.
-// The launch's op offsets and the block descriptors are first staged in LDS
-// (when they fit), so a thread finds its op and its arrays without a chain of
-// dependent global loads.
-constexpr int kOpsInLds = 256;
-constexpr int kBlocksInLds = 64;
-
-__global__ __launch_bounds__(256) void k_ops(const DevBlock* blocks, int n_blocks, const DevOp* ops, int op_lo,
-                                             int op_hi, long long total, int slot, int src, int props) {
-  __shared__ long long s_begin[kOpsInLds];
-  __shared__ DevBlock s_blocks[kBlocksInLds];
-  const int n_ops = op_hi - op_lo;
-  const bool ops_lds = n_ops <= kOpsInLds, blk_lds = n_blocks <= kBlocksInLds;
-  const long long base = ops[op_lo].begin;
-  if (ops_lds)
-    for (int t = threadIdx.x; t < n_ops; t += 256) s_begin[t] = ops[op_lo + t].begin - base;
-  if (blk_lds) {
-    static_assert(sizeof(DevBlock) % 8 == 0, "DevBlock is copied as 8-byte words");
-    const int words = n_blocks * (int)(sizeof(DevBlock) / 8);
-    const long long* src_w = reinterpret_cast<const long long*>(blocks);
-    long long* dst_w = reinterpret_cast<long long*>(s_blocks);
-    for (int w = threadIdx.x; w < words; w += 256) dst_w[w] = src_w[w];
-  }
-  __syncthreads();
-  const long long gid = blockIdx.x * 256ll + threadIdx.x;
-  if (gid >= total) return;
-  int lo = 0, hi = n_ops - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    const long long b = ops_lds ? s_begin[mid] : ops[op_lo + mid].begin - base;
-    if (b <= gid) lo = mid; else hi = mid - 1;
-  }
-  const DevOp op = ops[op_lo + lo];
-  op_point(blk_lds ? s_blocks : blocks, op, gid - (op.begin - base), slot, src, props != 0);
+// One launch of independent ops.  A workgroup belongs to one op, so the op and
+// its block come by scalar loads at once; the launches are chains of dependent
+// loads and little else (16x16x16 cells: 4.3 us; with a
+// binary search over the ops by every lane and the blocks staged through LDS
+// 7.4 us).
+template <bool FACE_STATE>
+__global__ __launch_bounds__(kOpWg) void k_ops(const DevBlock* blocks, const DevOp* ops, const OpWg* wgs, int slot,
+                                               int src, int props) {
+  const OpWg w = wgs[blockIdx.x];
+  op_item<FACE_STATE>(blocks, ops[w.op], w.first + (int)threadIdx.x, slot, src, props != 0);
 }
 
 // store_last_step and compute_square_of_dbv + reduction_of_dv_squared<4>
@@ -615,12 +588,11 @@ void padded_pass(const DevBlock& B, int slot, int what, hipStream_t st, long lon
   *n += 1;
 }
 
-void ops_launch(const DevBlock* d_blocks, int n_blocks, const DevOp* d_ops, int op_lo, int op_hi, long long total, int slot,
-                int src, hipStream_t st, long long* n, bool props) {
-  if (total <= 0) return;
-  const unsigned nb = (unsigned)((total + 255) / 256);
-  hipLaunchKernelGGL(k_ops, dim3(nb), dim3(256), 0, st, d_blocks, n_blocks, d_ops, op_lo, op_hi, total, slot, src,
-                     props ? 1 : 0);
+void ops_launch(const DevBlock* blocks, const DevOp* ops, const OpWg* wgs, int n_wg, bool face_state, int slot, int src,
+                bool props, hipStream_t st, long long* n) {
+  if (n_wg <= 0) return;
+  if (face_state) hipLaunchKernelGGL(k_ops<true>, dim3(n_wg), dim3(kOpWg), 0, st, blocks, ops, wgs, slot, src, props);
+  else hipLaunchKernelGGL(k_ops<false>, dim3(n_wg), dim3(kOpWg), 0, st, blocks, ops, wgs, slot, src, props);
   *n += 1;
 }
 

@@ -5,9 +5,6 @@
 
 namespace ostc {
 
-template <class T>
-using gptr = __attribute__((address_space(1))) T*;
-
 // What one stage reads and writes of a block, with the arrays as pointers
 // into global memory.  The block table is itself read from memory, so the
 // pointers it holds are generic to the compiler, which would then access
