@@ -796,7 +796,9 @@ int batched_record(ostc_ctx c, long long* n, int ev_base) {
   }
   if (!c->s.fixed_time_step) {
     FusedArgs a = fused_args(c, 0, 1, 0);
-    dt_rows(a, (int)c->blocks.size(), c->cus * 4, c->d_dt, c->st, n);
+    long long cells = 0;
+    for (auto& B : c->blocks) cells = std::max(cells, B.d.n0);
+    dt_rows(a, (int)c->blocks.size(), cells, c->cus * 16, c->d_dt, c->st, n);
   }
   for (int rk = 0; rk < 3; ++rk) {
     const int r = batched_stage(c, rk, n, ev_base);

@@ -72,7 +72,9 @@ bool sweep_scheme(int scheme);    // component-wise WENO: 50, 51, 71
 int sweep_valid(int scheme);      // padded points a wave of the x sweep advances by
 int visc_cells_per_wg();          // ... and a workgroup of the viscous kernel
 void sweep_launch(const FusedArgs& a, const SweepPlan& s, bool update, hipStream_t st, long long* n);
-void dt_rows(const FusedArgs& a, int n_blocks, int n_wg, double* dt_bits, hipStream_t st, long long* n);
+// about n_wg workgroups over all blocks; max_cells: interior nodes of the largest
+void dt_rows(const FusedArgs& a, int n_blocks, long long max_cells, int n_wg, double* dt_bits, hipStream_t st,
+             long long* n);
 
 // reverse mode, ostc_kernels_adjoint.hip
 struct VjpArgs {

@@ -593,22 +593,24 @@ __device__ double local_dt_point_f(const StageBlock& B, const Params& P, int p) 
 
 __global__ void k_dt_init(unsigned long long* bits) { *bits = (unsigned long long)__double_as_longlong(1e6); }
 
-// Every block's interior walked row by row (consecutive lanes, consecutive i:
-// whole cache lines of the metric and primitive planes; tiles would read
-// 16-double pieces of rows that straddle lines), grid-stride over the cells of
-// one block after another.
-__global__ __launch_bounds__(256) void k_dt_rows(FusedArgs A, int n_blocks, unsigned long long* bits) {
+// Block blockIdx.y's interior walked row by row (consecutive lanes, consecutive
+// i: whole cache lines of the metric and primitive planes; tiles would read
+// 16-double pieces of rows that straddle lines).  The grid is cut to the
+// blocks: atomics at one address wait for one another, so a workgroup without
+// cells issues none and one whose minimum is no longer the least skips it
+// (1024 workgroups took 14 us for 16^3 cells), and workgroups that take the
+// blocks in turn wait for each block's loads (12 blocks of 12^3: 25 us).
+__global__ __launch_bounds__(256) void k_dt_rows(FusedArgs A, unsigned long long* bits) {
   __shared__ double part[4];
   const int tid = threadIdx.x;
   double v = 1e6;
   const unsigned stride = gridDim.x * 256u;
-  for (int b = 0; b < n_blocks; ++b) {
-    const StageBlock B = stage_block(A.blocks[b], 0, 0);  // the step's state, slot 0
-    const unsigned row = (unsigned)B.mx, plane = row * (unsigned)B.my, n = plane * (unsigned)B.mz;
-    for (unsigned q = blockIdx.x * 256u + tid; q < n; q += stride) {
-      const unsigned k = q / plane, r = q - k * plane, j = r / row, i = r - j * row;
-      v = fmin(v, local_dt_point_f(B, A.P, poff(B, (int)i, (int)j, (int)k)));
-    }
+  const StageBlock B = stage_block(A.blocks[blockIdx.y], 0, 0);  // the step's state, slot 0
+  const unsigned row = (unsigned)B.mx, plane = row * (unsigned)B.my, n = plane * (unsigned)B.mz;
+  if (blockIdx.x * 256u >= n) return;
+  for (unsigned q = blockIdx.x * 256u + tid; q < n; q += stride) {
+    const unsigned k = q / plane, r = q - k * plane, j = r / row, i = r - j * row;
+    v = fmin(v, local_dt_point_f(B, A.P, poff(B, (int)i, (int)j, (int)k)));
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v = fmin(v, __shfl_xor(v, off, 64));
@@ -617,7 +619,8 @@ __global__ __launch_bounds__(256) void k_dt_rows(FusedArgs A, int n_blocks, unsi
   if (tid == 0) {
     for (int w = 1; w < 4; ++w) v = fmin(v, part[w]);
     v = fmin(v, part[0]);
-    atomicMin(bits, (unsigned long long)__double_as_longlong(v));
+    const unsigned long long mine = (unsigned long long)__double_as_longlong(v);
+    if (mine < __hip_atomic_load(bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(bits, mine);
   }
 }
 
@@ -722,10 +725,12 @@ int fused_lds_bytes(int scheme, int index) {
   return -1;
 }
 
-void dt_rows(const FusedArgs& a, int n_blocks, int n_wg, double* dt_bits, hipStream_t st, long long* n) {
+void dt_rows(const FusedArgs& a, int n_blocks, long long max_cells, int n_wg, double* dt_bits, hipStream_t st,
+             long long* n) {
+  const long long nx = std::min<long long>((max_cells + 255) / 256, std::max(1, n_wg / n_blocks));
   auto* bits = reinterpret_cast<unsigned long long*>(dt_bits);
   hipLaunchKernelGGL(k_dt_init, dim3(1), dim3(1), 0, st, bits);
-  hipLaunchKernelGGL(k_dt_rows, dim3(n_wg), dim3(256), 0, st, a, n_blocks, bits);
+  hipLaunchKernelGGL(k_dt_rows, dim3((unsigned)nx, n_blocks), dim3(256), 0, st, a, bits);
   *n += 2;
 }
 
