@@ -105,7 +105,7 @@ struct ostc_ctx_s {
   std::vector<Group> bc_rounds, comm_levels;
   Group props, rim;
   std::vector<std::vector<Group>> plain_bc;  // one block's boundary ops
-  std::vector<std::vector<int>> bc_order;    // the same ops in the reference's order
+  std::vector<std::vector<Group>> adj_bc;    // the launches of their transposes
   std::vector<Group> plain_comm;             // one inner face each, in the reference's order
   int tile_index = 0, n_wg = 0, xcd_remap = 1, n_tiles = 0, waves = 0, split = 0;
   int* d_tile_block = nullptr;
@@ -417,7 +417,7 @@ int build_ops(ostc_ctx c) {
   c->comm_levels.clear();
   c->plain_comm.clear();
   c->plain_bc.assign(nb, {});
-  c->bc_order.assign(nb, {});
+  c->adj_bc.assign(nb, {});
   std::vector<OpWg> wgs;
   // one launch of the ops added by f
   auto group = [&](auto f) {
@@ -437,8 +437,9 @@ int build_ops(ostc_ctx c) {
     c->ops.push_back(o);
   };
   int levels = 0;
+  std::vector<std::vector<int>> index(nb);  // of a block's boundary ops in c->ops
   for (int b = 0; b < nb; ++b) {
-    c->bc_order[b].resize(bc_of_block[b].size());
+    index[b].resize(bc_of_block[b].size());
     for (auto& o : bc_of_block[b]) levels = std::max(levels, o.level + 1);
   }
   for (int L = 0; L < levels; ++L)
@@ -447,13 +448,35 @@ int build_ops(ostc_ctx c) {
         const Group g = group([&] {
           for (size_t q = 0; q < bc_of_block[b].size(); ++q)
             if (bc_of_block[b][q].level == L) {
-              c->bc_order[b][q] = (int)c->ops.size();
+              index[b][q] = (int)c->ops.size();
               add(bc_of_block[b][q].op);
             }
         });
         if (g.hi > g.lo) c->plain_bc[b].push_back(g);
       }
     }));
+  // The transposes of the copies, in the reverse order: a transpose writes what
+  // the copy reads too, so two that read the same cells conflict as well.
+  for (int b = 0; b < nb; ++b) {
+    std::vector<LeveledOp> t;
+    std::vector<int> at;
+    for (size_t q = bc_of_block[b].size(); q-- > 0;) {
+      LeveledOp o = bc_of_block[b][q];
+      if (o.op.type != OP_BC_OUTFLOW && o.op.type != OP_BC_PERIODIC) continue;
+      o.w.insert(o.w.end(), o.r.begin(), o.r.end());
+      o.level = level_after(t, t.size(), o);
+      t.push_back(o);
+      at.push_back(index[b][q]);
+    }
+    int n = 0;
+    for (auto& o : t) n = std::max(n, o.level + 1);
+    for (int L = 0; L < n; ++L)
+      c->adj_bc[b].push_back(group([&] {
+        for (size_t q = 0; q < t.size(); ++q)
+          for (long long first = 0; t[q].level == L && first < t[q].op.count; first += kOpWg)
+            wgs.push_back(OpWg{at[q], (int)first});
+      }));
+  }
   levels = bulk.empty() ? 0 : 1;
   for (auto& e : edge) levels = std::max(levels, e.level + 1);
   for (int L = 0; L < levels; ++L)
@@ -1786,10 +1809,10 @@ int restore_state(ostc_ctx c, const DevBlock& B, const double* from) {
   return OSTC_OK;
 }
 
-// Transposed boundary copies of block b, in the reverse of their order.
+// Transposed boundary copies of block b.
 void bc_transpose(ostc_ctx c, int b, double* lam) {
   const DevBlock& B = c->blocks[b].d;
-  for (auto it = c->bc_order[b].rbegin(); it != c->bc_order[b].rend(); ++it) adj_bc_op(B, c->ops[*it], lam, c->st);
+  for (const Group& g : c->adj_bc[b]) adj_bc_ops(B, c->d_ops, c->d_op_wg + g.wg_lo, g.n_wg, lam, c->st);
 }
 
 }  // namespace

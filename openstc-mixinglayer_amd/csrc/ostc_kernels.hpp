@@ -99,7 +99,7 @@ void rhs_vjp(const VjpArgs& a, hipStream_t st, long long* n);
 void adj_stage_pre(const DevBlock& B, double* lam, double* lam_qn, double* w, double ra, double rb, double cdt,
                    hipStream_t st);
 void adj_stage_qn(const DevBlock& B, double* lam, double* lam_qn, hipStream_t st);
-void adj_bc_op(const DevBlock& B, const DevOp& op, double* lam, hipStream_t st);
+void adj_bc_ops(const DevBlock& B, const DevOp* ops, const OpWg* wgs, int n_wg, double* lam, hipStream_t st);
 
 constexpr int kMaxModes = 64;
 struct FourierModes {        // see ostc_fourier in abi.h

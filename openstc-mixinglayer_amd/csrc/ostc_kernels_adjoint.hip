@@ -525,32 +525,46 @@ __global__ __launch_bounds__(kT) void k_stage_qn(Geo G, double* lam, double* lam
   }
 }
 
-// Transpose of one boundary op (ghost = copy of a source cell):
-// lam[src] += lam[ghost], lam[ghost] = 0.  Sources and ghosts of one op are
-// disjoint, and the ghosts sharing a source belong to one thread.
-__global__ __launch_bounds__(kT) void k_bc_adj(Geo G, DevOp op, double* lam) {
-  const long long t = (long long)blockIdx.x * kT + threadIdx.x;
-  if (t >= op.count) return;
-  const int i = op.lo[0] + (int)(t % op.n[0]);
-  const int j = op.lo[1] + (int)((t / op.n[0]) % op.n[1]);
-  const int k = op.lo[2] + (int)(t / ((long long)op.n[0] * op.n[1]));
-  int d[3] = {0, 0, 0};
-  d[op.axis] = op.side;
-  int so[3] = {i, j, k};
-  if (op.type == OP_BC_PERIODIC) {
-    const int m = op.axis == 0 ? G.mx : (op.axis == 1 ? G.my : G.mz);
-    so[op.axis] = op.side < 0 ? m - 1 : 0;
-  }
-  for (int g = 1; g <= G.g; ++g) {
-    const long long pg = gidx(G, i + g * d[0], j + g * d[1], k + g * d[2]);
-    const long long ps = op.type == OP_BC_PERIODIC ? gidx(G, so[0] + g * d[0], so[1] + g * d[1], so[2] + g * d[2])
-                                                   : gidx(G, i, j, k);
+// Transpose of boundary ops (ghost = copy of a source cell) on one component
+// a lane: lam[src] += lam[ghost], lam[ghost] = 0.  Sources and ghosts of the
+// ops of one launch are disjoint, and the ghosts sharing a source belong to one
+// lane.  A lane has everything it reads in flight before its first store (one
+// op, point and all its ghosts and components a lane: 10.4 us a launch of one
+// face of 48^3 cells; 5.5 us of two faces).
+__global__ __launch_bounds__(kOpWg) void k_bc_adj(Geo G, const DevOp* ops, const OpWg* wgs, double* lam) {
+  const OpWg w = wgs[blockIdx.x];
+  const DevOp& op = ops[w.op];
+  const int t = w.first + (int)threadIdx.x;
+  if (t >= op.n[0] * op.n[1] * op.n[2]) return;
+  const int u = t / op.n[0], v = u / op.n[1];
+  const int i = op.lo[0] + t - u * op.n[0], j = op.lo[1] + u - v * op.n[1], k = op.lo[2] + v;
+  const int axis = op.axis, side = op.side;
+  const int di = axis == 0 ? side : 0, dj = axis == 1 ? side : 0, dk = axis == 2 ? side : 0;
+  double* x = lam + blockIdx.y * G.sz;
+  double ghost[kMaxGhost];
 #pragma unroll
-    for (int l = 0; l < 5; ++l) {
-      lam[ps + l * G.sz] += lam[pg + l * G.sz];
-      lam[pg + l * G.sz] = 0;
-    }
+  for (int g = 1; g <= kMaxGhost; ++g)
+    if (g <= G.g) ghost[g - 1] = x[gidx(G, i + g * di, j + g * dj, k + g * dk)];
+  if (op.type == OP_BC_PERIODIC) {
+    const int m = axis == 0 ? G.mx : (axis == 1 ? G.my : G.mz), from = side < 0 ? m - 1 : 0;
+    const int si = axis == 0 ? from : i, sj = axis == 1 ? from : j, sk = axis == 2 ? from : k;
+    double sum[kMaxGhost];
+#pragma unroll
+    for (int g = 1; g <= kMaxGhost; ++g)
+      if (g <= G.g) sum[g - 1] = x[gidx(G, si + g * di, sj + g * dj, sk + g * dk)] + ghost[g - 1];
+#pragma unroll
+    for (int g = 1; g <= kMaxGhost; ++g)
+      if (g <= G.g) x[gidx(G, si + g * di, sj + g * dj, sk + g * dk)] = sum[g - 1];
+  } else {
+    double sum = x[gidx(G, i, j, k)];
+#pragma unroll
+    for (int g = 1; g <= kMaxGhost; ++g)
+      if (g <= G.g) sum += ghost[g - 1];
+    x[gidx(G, i, j, k)] = sum;
   }
+#pragma unroll
+  for (int g = 1; g <= kMaxGhost; ++g)
+    if (g <= G.g) x[gidx(G, i + g * di, j + g * dj, k + g * dk)] = 0;
 }
 
 // ------------------------------------------------- differentiation workload
@@ -726,9 +740,8 @@ void adj_stage_qn(const DevBlock& B, double* lam, double* lam_qn, hipStream_t st
   k_stage_qn<<<blocks_for(B.n0), kT, 0, st>>>(geo_of(B), lam, lam_qn);
 }
 
-void adj_bc_op(const DevBlock& B, const DevOp& op, double* lam, hipStream_t st) {
-  if (op.type != OP_BC_OUTFLOW && op.type != OP_BC_PERIODIC) return;
-  k_bc_adj<<<blocks_for(op.count), kT, 0, st>>>(geo_of(B), op, lam);
+void adj_bc_ops(const DevBlock& B, const DevOp* ops, const OpWg* wgs, int n_wg, double* lam, hipStream_t st) {
+  k_bc_adj<<<dim3(n_wg, 5), kOpWg, 0, st>>>(geo_of(B), ops, wgs, lam);
 }
 
 void fourier_add(const DevBlock& B, const FourierModes& F, double* bv, hipStream_t st) {

@@ -41,6 +41,9 @@ struct DevOp {
   const unsigned long long* pass;  // OP_BC_INFLOW: boundary-condition passes per block so far
 };
 
+// Largest ngg (WENO-Z7).
+constexpr int kMaxGhost = 4;
+
 // A workgroup of a launch: its op and its first item (point and layer).
 struct OpWg { int op, first; };
 constexpr int kOpWg = 256;
