@@ -307,20 +307,18 @@ def reacting_cpu_baseline(tables, n, steps, spatial=False):
                       f"layer, {dt:.1f} s on {threads} OpenMP threads"}
 
 
-def measured_traffic(tile, split: int, waves: int):
-    """HBM bytes per launch of the fused kernel for this tile configuration,
-    from the FETCH_SIZE / WRITE_SIZE counter runs summarised in
-    profiles/fused_rhs_update_batched24_pmc.txt (the same 24-block case), or
-    None when the configuration was not measured."""
+def measured_traffic():
+    """HBM bytes of one stage's kernels (x sweep, y and z marches, viscous +
+    update) on the 24-block case, from the FETCH_SIZE / WRITE_SIZE counter runs
+    summarised in profiles/fused_rhs_update_batched24_pmc.txt, or None."""
     path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "profiles",
                         "fused_rhs_update_batched24_pmc.txt")
-    if waves != 0 or not os.path.exists(path):
+    if not os.path.exists(path):
         return None
-    want = f"traffic tile={tile[0]}x{tile[1]}x{tile[2]} split={int(split)} "
     with open(path) as f:
         for line in f:
-            if line.startswith(want):
-                fields = dict(kv.split("=") for kv in line.split()[1:])
+            if line.startswith("traffic stage "):
+                fields = dict(kv.split("=") for kv in line.split()[2:])
                 return int(fields["bytes"])
     return None
 
@@ -355,14 +353,14 @@ def fused_roofline(cells, avg_kernel_ms, rate_mcells, tile_index, tile_split, ti
     hbm_bound = HBM_PEAK_GBS * 1e9 / bytes_per_launch < FP64_PEAK_TFLOPS * 1e12 / flops_per_launch
     b_step = 3 * BYTES_PER_CELL_STAGE + 8 * 5
     step_roof = min(HBM_PEAK_GBS * 1e9 / b_step, FP64_PEAK_TFLOPS * 1e12 / f["step_per_cell"]) / 1e6
-    traffic = measured_traffic(pkg.tile_shapes()[tile_index], tile_split, tile_waves)
+    traffic = measured_traffic()
     hbm = {"achieved": gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": gbs / HBM_PEAK_GBS}
     fp64 = {"achieved": tfs, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": tfs / FP64_PEAK_TFLOPS}
     main = hbm if hbm_bound else fp64
     return {"bound": "hbm" if hbm_bound else "fp64", **main, "traffic": traffic,
             "traffic_source": "profiles/fused_rhs_update_batched24_pmc.txt (rocprofv3 FETCH_SIZE + WRITE_SIZE, "
                               "copy-calibrated, bytes per launch)" if traffic else None,
-            "kernel": "k_fused (RHS+update, one RK stage over all blocks)",
+            "kernel": "k_sweep_x, k_sweep_march<1|2>, k_visc_update_rows (RHS+update, one RK stage over all blocks)",
             "hbm": hbm, "fp64": fp64,
             "algorithmic_bytes_per_launch": bytes_per_launch, "algorithmic_flops_per_launch": flops_per_launch,
             "flops_source": "profiles/flops_per_cell_air.txt (oracle on a counting scalar; fp64 vector peak)",

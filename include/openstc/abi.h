@@ -322,8 +322,8 @@ int ostc_apply_bc(ostc_ctx ctx, int block);                   /* DBoundCond::app
 int ostc_exchange(ostc_ctx ctx);                              /* data_communication, inner faces */
 int ostc_update_properties(ostc_ctx ctx, int block);          /* update_physical_properties<Air> */
 int ostc_copy_qn(ostc_ctx ctx, int block);                    /* qn <- cv (src/RK.cuh:99-102) */
-/* Batched fused RHS of one block written to dq (no update), for checking
- * the fused kernel's residual against the per-direction kernels. */
+/* Batched RHS of one block written to dq (no update), for checking the batched
+ * kernels' residual against the per-direction kernels. */
 int ostc_batched_rhs(ostc_ctx ctx, int block);
 
 /* Residual norms sqrt(sum(dv^2)/N) of (rho, |V|, p, T) against the last
@@ -331,11 +331,13 @@ int ostc_batched_rhs(ostc_ctx ctx, int block);
 int ostc_store_last_step(ostc_ctx ctx);
 int ostc_residual(ostc_ctx ctx, double res[4]);
 
-/* Launch configuration of the fused kernel: tile index into the compiled
- * table, workgroups per CU of a persistent grid (0: one workgroup per tile),
- * and split = 1 to run each stage as an inviscid kernel followed by a
- * viscous + update kernel.  ostc_autotune times every combination on the
- * current blocks and keeps the fastest. */
+/* Launch configuration of the batched tile kernel (schemes 52 and 72): tile
+ * index into the compiled table, workgroups per CU of a persistent grid (0: one
+ * workgroup per tile), and split = 1 to run each stage as an inviscid kernel
+ * followed by a viscous + update kernel.  ostc_autotune times every
+ * combination on the current blocks and keeps the fastest.  The sweeps of
+ * schemes 50, 51 and 71 have no tile: for them the configuration is kept and
+ * reported but changes nothing. */
 int ostc_tile_count(int* n);
 int ostc_tile_shape(int index, int* tx, int* ty, int* tz);
 int ostc_set_tile(ostc_ctx ctx, int index, int waves_per_cu, int split);
@@ -560,9 +562,8 @@ typedef struct {
                                  relaxation rate is sigma; 0: the reference's term as written, without J
                                  (src/SpongeLayer.cu:155), whose rate is sigma / J */
 } ostc_sponge;
-/* Air contexts: the same sponge layer on the five conservative variables,
- * with OSTC_MODE_PLAIN and the stage operators (the fused batched kernel
- * refuses it); before ostc_finalize, per block, as ostc_fr_set_sponge. */
+/* Air contexts: the same sponge layer on the five conservative variables, in
+ * every mode; before ostc_finalize, per block, as ostc_fr_set_sponge. */
 int ostc_set_sponge(ostc_ctx ctx, int block, const ostc_sponge* sp, const double* x, const double* y,
                     const double* z);
 /* Before ostc_fr_finalize, per block: x, y, z are the block's node coordinates

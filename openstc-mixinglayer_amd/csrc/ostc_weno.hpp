@@ -19,9 +19,10 @@
 // not reach the leading digits, and the differences of neighbouring points are
 // exact or nearly so.  49 operations and four reciprocals a side, a reciprocal
 // being one estimate and three FMAs.
-// Step of 24 air blocks (12.5 M nodes, WENO-Z5) 16.25 -> 14.42 ms, WENO-Z7 on
-// 101x75x49 nodes 688 -> 603 us, characteristic 1.97 -> 1.78 ms, a reacting
-// 256x128x64 block 20.3 -> 19.5 ms.  The error of a step against 64-bit whole-array
+// By itself, in the tile kernels that then did every scheme: a step of 24 air
+// blocks (12.5 M nodes, WENO-Z5) 16.25 -> 14.42 ms, WENO-Z7 on 101x75x49 nodes
+// 688 -> 603 us, characteristic 1.97 -> 1.78 ms, a reacting 256x128x64 block
+// 20.3 -> 19.5 ms.  The error of a step against 64-bit whole-array
 // arithmetic in another order is no larger (7.2e-15 -> 6.9e-15 of v on 16^3).
 #pragma once
 #include <hip/hip_runtime.h>
