@@ -76,6 +76,18 @@ inline bool boundary_range(const int r[6], const int ext[3], int ngg, FaceRange*
   return true;
 }
 
+// The node that ghost layer g = 1..ngg of a periodic face takes, on an axis of
+// m >= 2 nodes of which the first and the last are one: m-1-g below node 0 and
+// g above node m-1.  On an axis of m <= ngg nodes that node is itself a ghost,
+// which the reference's loop over the layers has filled just before
+// (src/BoundCond.cuh:1443-1486); here it is the interior node that the chain
+// of copies ends at, so that no layer waits for another.
+constexpr int periodic_source(int m, int side, int g) {
+  int q = g - 1;
+  while (q >= m - 1) q -= m - 1;
+  return side < 0 ? m - 2 - q : 1 + q;
+}
+
 inline FaceMap aligned_face(int axis, int side, const int ext[3], const int text[3], int ngg, int target) {
   FaceMap m{};
   m.target = target;

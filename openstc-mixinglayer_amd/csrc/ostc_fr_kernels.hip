@@ -17,6 +17,7 @@
 
 #include <algorithm>
 
+#include "ostc_faces.hpp"
 #include "ostc_fr.hpp"
 #include "ostc_inflow.hpp"
 #include "ostc_weno.hpp"
@@ -487,10 +488,9 @@ __global__ __launch_bounds__(kT) void k_ghost(FrArgs A, const FrBlockDev* blocks
       break;
     }
     case GHOST_PERIODIC: {
-      const int g = layer + 1, m = axis == 0 ? B.mx : (axis == 1 ? B.my : B.mz), from = side < 0 ? m - 1 : 0;
-      const int si = axis == 0 ? from : i, sj = axis == 1 ? from : j, sk = axis == 2 ? from : k;
+      const int g = layer + 1, from = ostc::periodic_source(axis == 0 ? B.mx : (axis == 1 ? B.my : B.mz), side, g);
       put_node<NS>(A.T, N, pid(B, i + g * di, j + g * dj, k + g * dk),
-                   get_node<NS>(N, pid(B, si + g * di, sj + g * dj, sk + g * dk)));
+                   get_node<NS>(N, pid(B, axis == 0 ? from : i, axis == 1 ? from : j, axis == 2 ? from : k)));
       break;
     }
     case GHOST_INNER: {
