@@ -43,7 +43,8 @@ struct Tab : ostc_mech_tables {
 // temperature at which its polynomials are evaluated (not below t_low, beyond
 // which h continues linearly).  A wave whose lanes all lie in one range, as
 // nearly every wave does, reads the coefficients by scalar loads (range is the
-// same for the wave); a mixed wave selects them per lane.
+// same for the wave); a mixed wave selects them per lane.  A NaN temperature
+// stays one (fmax would make it t_low and every property finite).
 template <int NS, class F>
 __device__ __forceinline__ void each_species(const Tab* __restrict__ T, double t, F f) {
   if (__all(t >= T->mid_hi)) {
@@ -51,10 +52,10 @@ __device__ __forceinline__ void each_species(const Tab* __restrict__ T, double t
     for (int i = 0; i < NS; ++i) f(i, 1, t);
   } else if (__all(t < T->mid_lo)) {
 #pragma unroll
-    for (int i = 0; i < NS; ++i) f(i, 0, fmax(t, T->t_low[i]));
+    for (int i = 0; i < NS; ++i) f(i, 0, t < T->t_low[i] ? T->t_low[i] : t);
   } else {
 #pragma unroll
-    for (int i = 0; i < NS; ++i) f(i, t >= T->t_mid[i] ? 1 : 0, fmax(t, T->t_low[i]));
+    for (int i = 0; i < NS; ++i) f(i, t >= T->t_mid[i] ? 1 : 0, t < T->t_low[i] ? T->t_low[i] : t);
   }
 }
 
