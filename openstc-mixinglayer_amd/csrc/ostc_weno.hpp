@@ -29,40 +29,51 @@
 
 namespace ostc {
 
-// 1 / x for x in the range where 1 / x is normal: the hardware's estimate
-// (relative error measured 2^-24.4) and one cubic step.  Measured over 2^+-300: within 1.0 * 2^-53
-// of the exact value, as a correctly rounded quotient is.
-__device__ __forceinline__ double rcp64(double x) {
+// 1 / x for normal x whose reciprocal is normal: the hardware's estimate
+// (relative error measured 2^-24.4) and one cubic step.  Measured over
+// 2^+-300: within 1.0 * 2^-53 of the exact value, as a correctly rounded
+// quotient is.  A zero or infinite x gives NaN: only for operands that are
+// neither, or whose result is NaN by the divisions of the textbook form as
+// well (the smoothness indicators: eps and squares of flux differences, zero
+// only where eps is, infinite only beyond differences of 10^153).
+__device__ __forceinline__ double rcp64_normal(double x) {
   const double r = __builtin_amdgcn_rcp(x);
   const double e = __builtin_fma(-x, r, 1.0);
   return __builtin_fma(r, __builtin_fma(e, e, e), r);
 }
 
-// sqrt(x) for normal x > 0 (0 gives NaN): estimate (2^-24.2), one coupled
-// step for the root and half its reciprocal, one residual correction.
-// Measured over 2^+-300: within 1.0 * 2^-53 of the exact value.
+// The same with the result of a division for a zero, infinite or NaN x (one
+// instruction more).
+__device__ __forceinline__ double rcp64(double x) { return __builtin_amdgcn_div_fixup(rcp64_normal(x), x, 1.0); }
+
+// sqrt(x) for x that is no subnormal number: estimate (2^-24.2), one coupled
+// step for the root and half its reciprocal, one residual correction; 0 and
+// infinity are their own roots.  Measured over 2^+-300: within 1.0 * 2^-53 of
+// the exact value.
 __device__ __forceinline__ double sqrt64(double x) {
+  constexpr int zero_or_inf = 0x020 | 0x040 | 0x200;  // -0, +0, +infinity
   const double s = __builtin_amdgcn_rsq(x);
   const double h = x * s, g = 0.5 * s;
   const double d = __builtin_fma(-h, g, 0.5);
   const double h1 = __builtin_fma(h, d, h), g1 = __builtin_fma(g, d, g);
-  return __builtin_fma(__builtin_fma(-h1, h1, x), g1, h1);
+  const double root = __builtin_fma(__builtin_fma(-h1, h1, x), g1, h1);
+  return __builtin_amdgcn_class(x, zero_or_inf) ? x : root;
 }
 
-// n / d as an IEEE division rounds it, for operands and quotient of ordinary
-// magnitude: the compiler's own sequence for a division without its scaling,
-// fix-up and condition-code steps (estimate, two Newton steps, quotient and one
-// correction).
+// n / d as an IEEE division rounds it, for d and quotient that are no
+// subnormal numbers: the compiler's own sequence for a division without its
+// scaling and condition-code steps (estimate, two Newton steps, quotient and
+// one correction, fix-up of zeros, infinities and NaN).
 __device__ __forceinline__ double div64(double n, double d) {
   double r = __builtin_amdgcn_rcp(d);
   r = __builtin_fma(__builtin_fma(-d, r, 1.0), r, r);
   r = __builtin_fma(__builtin_fma(-d, r, 1.0), r, r);
   const double q = n * r;
-  return __builtin_fma(__builtin_fma(-d, q, n), r, q);
+  return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-d, q, n), r, q), d, n);
 }
 
-// n / d with r the correctly rounded 1 / d at hand: correctly rounded (Markstein
-// 1990) in three instructions.
+// n / d of a finite n with r the correctly rounded 1 / d of a normal d at hand:
+// correctly rounded (Markstein 1990) in three instructions.
 __device__ __forceinline__ double div64(double n, double d, double r) {
   const double q = n * r;
   return __builtin_fma(__builtin_fma(-d, q, n), r, q);
@@ -79,7 +90,7 @@ __device__ __forceinline__ double weno5_side(double f0, double f1, double f2, do
   const double b0 = __builtin_fma(t0, t0, __builtin_fma(c133 * s0, s0, eps4));
   const double b1 = __builtin_fma(t1, t1, __builtin_fma(c133 * s1, s1, eps4));
   const double b2 = __builtin_fma(t2, t2, __builtin_fma(c133 * s2, s2, eps4));
-  double g0 = rcp64(b0), g1 = rcp64(b1), g2 = rcp64(b2);
+  double g0 = rcp64_normal(b0), g1 = rcp64_normal(b1), g2 = rcp64_normal(b2);
   if constexpr (Z) {  // 1 + (tau / (eps + beta))^2
     const double tau = b0 - b2;
     g0 *= tau;
@@ -96,7 +107,7 @@ __device__ __forceinline__ double weno5_side(double f0, double f1, double f2, do
   const double a0 = 3.0 * g0;
   const double num = __builtin_fma(a0, s1 - s0, -2.0 * (g2 * (s1 - s2)));
   const double sum = __builtin_fma(6.0, g1, a0 + g2);
-  return __builtin_fma(num, rcp64(sum), __builtin_fma(2.0, c, b));
+  return __builtin_fma(num, rcp64_normal(sum), __builtin_fma(2.0, c, b));
 }
 
 // One side of WENO-Z7 from seven points, upwind first: the face value is
@@ -119,7 +130,7 @@ __device__ __forceinline__ double weno7_side(double f0, double f1, double f2, do
   const double b2 = beta(__builtin_fma(6.0, d3, -__builtin_fma(2.0, q2, q3)), q2, r2);
   const double b3 = beta(__builtin_fma(6.0, d3, __builtin_fma(-5.0, q3, 2.0 * q4)), __builtin_fma(2.0, q3, -q4), r3);
   const double tau = b0 - b3;
-  double g0 = tau * rcp64(b0), g1 = tau * rcp64(b1), g2 = tau * rcp64(b2), g3 = tau * rcp64(b3);
+  double g0 = tau * rcp64_normal(b0), g1 = tau * rcp64_normal(b1), g2 = tau * rcp64_normal(b2), g3 = tau * rcp64_normal(b3);
   g0 = __builtin_fma(g0, g0, 1.0);
   g1 = __builtin_fma(g1, g1, 1.0);
   g2 = __builtin_fma(g2, g2, 1.0);
@@ -129,7 +140,7 @@ __device__ __forceinline__ double weno7_side(double f0, double f1, double f2, do
   const double num = __builtin_fma(-3.0 * g0, p0, __builtin_fma(-a2, p1, a3 * (p2 - p1)));
   const double sum = __builtin_fma(12.0, g1, g0 + a2) + a3;
   const double base = __builtin_fma(6.0, d2, __builtin_fma(4.0, q1, 3.0 * r1));
-  return __builtin_fma(num, rcp64(sum), base);
+  return __builtin_fma(num, rcp64_normal(sum), base);
 }
 
 // Face value of F+ plus face value of F-.  5-point schemes: vp = F+ at
