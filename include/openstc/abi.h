@@ -102,7 +102,9 @@ typedef struct {
    *   sv   n_spec planes of mass fractions (mixture contexts; ignored for air)
    *   qn   n_var planes: the state at the start of the step (per-block steps);
    *        batched steps use the array as intermediate stage storage
-   *   dq   n_var planes, no ghosts
+   *   dq   n_var planes, no ghosts: written by the residual calls and the
+   *        per-block steps; batched steps leave it alone (but for the split
+   *        stage of the tile kernels, ostc_set_tile)
    *   mul  viscosity (air contexts: the state the batched step leaves)
    *   jac  Jacobian */
   double* cv;

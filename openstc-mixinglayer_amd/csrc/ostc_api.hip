@@ -535,6 +535,26 @@ int need_fused(ostc_ctx c) {
               "inviscid_scheme 1/2/3/4/6 run with OSTC_MODE_PLAIN and the stage operators only");
 }
 
+// The planes in which the sweeps of a batched stage hand dq to one another, 40
+// bytes a node.  ostc_finalize allocates them where there is room, so that the
+// first step does not; where there is none, per-block steps still run, and
+// the calls that run batched stages try again and report it.
+int need_residual(ostc_ctx c) {
+  if (!sweep_scheme(c->P.scheme) || c->blocks[0].d.res) return OSTC_OK;
+  size_t n = 0;
+  for (auto& B : c->blocks) n += 5 * (size_t)B.d.n0;
+  void* v = nullptr;
+  HIPCHK(c, hipMalloc(&v, n * sizeof(double)));
+  c->allocs.push_back(v);
+  n = 0;
+  for (auto& B : c->blocks) {
+    B.d.res = static_cast<double*>(v) + n;
+    n += 5 * (size_t)B.d.n0;
+  }
+  HIPCHK(c, hipStreamSynchronize(c->st));  // queued kernels read the block table
+  return upload_blocks(c);
+}
+
 int set_tiles(ostc_ctx c, int index, int n_wg) {
   const TileShape t = fused_shape(c->P.scheme, index);
   const int lds = fused_lds_bytes(c->P.scheme, index);
@@ -1238,6 +1258,10 @@ int ostc_finalize(ostc_ctx c) {
   c->cv_bar.assign(c->blocks.size(), nullptr);
   if (c->s.fixed_time_step) HIPCHK(c, hipMemcpy(c->d_dt, &c->s.dt, sizeof(double), hipMemcpyHostToDevice));
   if ((r = build_sweeps(c))) return r;
+  if (need_fused(c) != OSTC_OK || need_residual(c) != OSTC_OK) {
+    (void)hipGetLastError();
+    c->err.clear();
+  }
   c->finalized = true;
   return set_tiles(c, 0, 0);
 }
@@ -1377,7 +1401,7 @@ int ostc_step(ostc_ctx c, int n_steps, int mode, double* last_dt) {
       if (r) return r;
     }
   } else if (mode == OSTC_MODE_BATCHED) {
-    if ((r = need_fused(c))) return r;
+    if ((r = need_fused(c)) || (r = need_residual(c))) return r;
     if (!c->graph_valid) {
       r = build_graph(c);
       if (r) return r;
@@ -1387,7 +1411,7 @@ int ostc_step(ostc_ctx c, int n_steps, int mode, double* last_dt) {
     if (last_dt && !c->s.fixed_time_step)
       HIPCHK(c, hipMemcpyAsync(&dt, c->d_dt, sizeof(double), hipMemcpyDeviceToHost, c->st));
   } else if (mode == OSTC_MODE_BATCHED_TIMED) {
-    if ((r = need_fused(c))) return r;
+    if ((r = need_fused(c)) || (r = need_residual(c))) return r;
     while ((long long)c->evpool.size() < 6ll * n_steps) {
       hipEvent_t e;
       HIPCHK(c, hipEventCreate(&e));
@@ -1676,7 +1700,7 @@ int ostc_tile_config(ostc_ctx c, int* index, int* waves_per_cu, int* split) {
 int ostc_autotune(ostc_ctx c, int reps, int* best_index, double* best_ms) {
   int r = check_ready(c);
   if (r) return r;
-  if ((r = need_fused(c))) return r;
+  if ((r = need_fused(c)) || (r = need_residual(c))) return r;
   if (reps < 1) reps = 3;
   double best = 1e30;
   int bi = c->tile_index, bw = 0, bs = 0;
@@ -1954,6 +1978,7 @@ int ostc_adjoint_forward(ostc_ctx c, int n_steps, int every, const ostc_theta* t
   r = check_theta(c, B, t);
   if (!r) r = adj_common(c);
   if (r) return r;
+  if ((r = need_residual(c))) return r;
   const size_t plane = 12 * (size_t)B.sz;
   const int n_seg = (n_steps + every - 1) / every;
   const int seg_len = std::min(every, n_steps);

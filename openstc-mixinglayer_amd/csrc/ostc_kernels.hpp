@@ -51,6 +51,7 @@ struct FusedArgs {
   Params P;
   int xcd_remap;             // 1: contiguous tile chunks per XCD
   int target_block;          // >= 0: only this block's tiles (dq mode)
+  int to_dq;                 // sweeps: the residual goes to the block's dq instead of res (sweep_launch)
 };
 
 struct TileShape { int tx, ty, tz, waves_per_eu; };  // waves_per_eu: occupancy hint given to the compiler
@@ -71,7 +72,7 @@ struct SweepPlan { const SweepItem* items[4]; int n[4]; };
 bool sweep_scheme(int scheme);    // component-wise WENO: 50, 51, 71
 int sweep_valid(int scheme);      // padded points a wave of the x sweep advances by
 int visc_cells_per_wg();          // ... and a workgroup of the viscous kernel
-void sweep_launch(const FusedArgs& a, const SweepPlan& s, bool update, hipStream_t st, long long* n);
+void sweep_launch(FusedArgs a, const SweepPlan& s, bool update, hipStream_t st, long long* n);
 // about n_wg workgroups over all blocks; max_cells: interior nodes of the largest
 void dt_rows(const FusedArgs& a, int n_blocks, long long max_cells, int n_wg, double* dt_bits, hipStream_t st,
              long long* n);

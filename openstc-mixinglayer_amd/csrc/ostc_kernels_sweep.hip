@@ -2,7 +2,10 @@
 // block of a batched stage (WENO5-JS 50, WENO-Z5 51, WENO-Z7 71) as three
 // sweeps without workgroup barriers: dq = s - dFx, then dq -= dFy, then
 // dq -= dFz, in the reference's order (src/RK.cuh:113-139), s the sponge term;
-// then the viscous fluxes and the RK update.
+// then the viscous fluxes and the RK update.  A step leaves the block's dq
+// array alone: between the kernels dq lies in planes of its own (a.to_dq: in
+// the array).  In the primitives of the slot that the stage writes, which are
+// free until then, its rows would be padded, and cut lines: 24 blocks 2 % slower.
 //
 // One tile kernel per stage did all of this with dq in registers (24 blocks,
 // 12.5 M nodes: 4.5 ms a stage).  It moved the fewest bytes, but it waited half
@@ -83,7 +86,7 @@ __global__ __launch_bounds__(256) void k_sweep_x(FusedArgs A, const SweepItem* i
   const StageBlock B = stage_block(A.blocks[it.block], A.in, A.out);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int n = B.sx * B.my * B.mz;
-  const int q = it.first + wave * VALID + lane, qc = min(q, n - 1);
+  const int qf = it.first + wave * VALID + lane, qc = min(qf, n - 1);
   const int row = qc / B.sx, ii = qc - row * B.sx, k = row / B.my, j = row - k * B.my, i = ii - B.g;
   const int o = poff(B, i, j, k);
   double(*L)[64] = lds[wave];
@@ -119,7 +122,8 @@ __global__ __launch_bounds__(256) void k_sweep_x(FusedArgs A, const SweepItem* i
     const double f = weno_face<SCHEME>(vp, vm, e[l == 0 ? 0 : (l == 4 ? 2 : 1)]);
     diff[l] = f - __shfl_up(f, 1, 64);
   }
-  if (lane < R || lane > 63 - R || q >= n || i < 0 || i >= B.mx) return;
+  if (lane < R || lane > 63 - R || qf >= n || i < 0 || i >= B.mx) return;
+  const gptr<double> res = A.to_dq ? B.dq : B.res;
   const int q0 = (k * B.my + j) * B.mx + i, n0 = (int)B.n0, s = B.sz;
   if (B.sp_sigma) {
     // sponge_layer_source (src/SpongeLayer.cu:68-160), the first term of the
@@ -127,10 +131,10 @@ __global__ __launch_bounds__(256) void k_sweep_x(FusedArgs A, const SweepItem* i
     const double sigma = B.sp_jac ? B.sp_sigma[q0] * B.jac[o] : B.sp_sigma[q0];
 #pragma unroll
     for (int l = 0; l < 5; ++l)
-      B.dq[q0 + l * n0] = (0.0 - sigma * (B.cvi[o + l * s] - B.sp_mean[q0 + l * n0])) - diff[l];
+      res[q0 + l * n0] = (0.0 - sigma * (B.cvi[o + l * s] - B.sp_mean[q0 + l * n0])) - diff[l];
   } else {
 #pragma unroll
-    for (int l = 0; l < 5; ++l) st(B.dq + l * n0, 8u * (unsigned)q0, 0.0 - diff[l]);
+    for (int l = 0; l < 5; ++l) st(res + l * n0, 8u * (unsigned)q0, 0.0 - diff[l]);
   }
 }
 
@@ -146,6 +150,7 @@ __global__ __launch_bounds__(64, 2) void k_sweep_march(FusedArgs A, const SweepI
   const SweepItem it = items[blockIdx.x];
   if (A.target_block >= 0 && it.block != A.target_block) return;
   const StageBlock B = stage_block(A.blocks[it.block], A.in, A.out);
+  const gptr<double> res = A.to_dq ? B.dq : B.res;
   const int third = D == 1 ? B.mz : B.my, n0 = (int)B.n0;
   const int col = it.first + (int)threadIdx.x, cc = min(col, B.mx * third - 1);
   const bool store = col == cc;
@@ -209,13 +214,13 @@ __global__ __launch_bounds__(64, 2) void k_sweep_march(FusedArgs A, const SweepI
   for (int c = 0; c < it.n; ++c) {
     double dq[5];
 #pragma unroll
-    for (int l = 0; l < 5; ++l) dq[l] = ld(B.dq + l * n0, 8u * (unsigned)q);
+    for (int l = 0; l < 5; ++l) dq[l] = ld(res + l * n0, 8u * (unsigned)q);
     advance(c + 1 < it.n);
     double f[5];
     face(f);
 #pragma unroll
     for (int l = 0; l < 5; ++l) {
-      if (store) st(B.dq + l * n0, 8u * (unsigned)q, dq[l] - (f[l] - left[l]));
+      if (store) st(res + l * n0, 8u * (unsigned)q, dq[l] - (f[l] - left[l]));
       left[l] = f[l];
     }
     q += dstep;
@@ -354,9 +359,9 @@ __device__ __forceinline__ void stage_update(const FusedArgs& A, const StageBloc
 
 // Viscous fluxes of all three directions added to the stored inviscid dq
 // (VISC), then the RK update of ring slot `out`; UPDATE false: dq is written
-// back instead.  As in the x sweep a wave takes 64 consecutive padded points
-// of the interior rows, one cell a lane: the x face is shared with the
-// neighbouring lane (62 of 64 update), the two y and the two z faces are
+// to the block's array instead.  As in the x sweep a wave takes 64 consecutive
+// padded points of the interior rows, one cell a lane: the x face is shared with
+// the neighbouring lane (62 of 64 update), the two y and the two z faces are
 // formed here.  u, v, w, T of the nine rows of the cells' yz cross section are
 // loaded at once into the wave's own LDS words (held in registers they spill:
 // 82 of 256), from which each face reads what it needs, x neighbours
@@ -376,11 +381,12 @@ __global__ __launch_bounds__(64 * kVWaves, 2) void k_visc_update_rows(FusedArgs 
   const int row = qc / B.sx, i = qc - row * B.sx - B.g, k = row / B.my, j = row - k * B.my;
   const bool store = lane > 0 && lane < 63 && qf < n && i >= 0 && i < B.mx;
   const int sy = B.sx, sz = B.sx * B.sy, o = poff(B, i, j, k);
+  const gptr<double> res = UPDATE ? B.res : B.dq;
   const int q = (k * B.my + j) * B.mx + i;
   double dq[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
   if (store) {
 #pragma unroll
-    for (int l = 0; l < 5; ++l) dq[l] = ld(B.dq + l * n0, 8u * (unsigned)q);
+    for (int l = 0; l < 5; ++l) dq[l] = ld(res + l * n0, 8u * (unsigned)q);
   }
   double jac = 1.0;
   if constexpr (VISC) {
@@ -445,7 +451,7 @@ __global__ __launch_bounds__(64 * kVWaves, 2) void k_visc_update_rows(FusedArgs 
     stage_update(A, B, o, *A.dt, jac, dq);
   } else {
 #pragma unroll
-    for (int l = 0; l < 5; ++l) st(B.dq + l * n0, 8u * (unsigned)q, dq[l]);
+    for (int l = 0; l < 5; ++l) st(res + l * n0, 8u * (unsigned)q, dq[l]);
   }
 }
 
@@ -462,7 +468,8 @@ bool sweep_scheme(int scheme) { return scheme == 50 || scheme == 51 || scheme ==
 
 int sweep_valid(int scheme) { return 64 - 2 * (scheme == 71 ? Stencil<71>::R : Stencil<51>::R); }
 
-void sweep_launch(const FusedArgs& a, const SweepPlan& s, bool update, hipStream_t st, long long* n) {
+void sweep_launch(FusedArgs a, const SweepPlan& s, bool update, hipStream_t st, long long* n) {
+  a.to_dq = !update;
   if (a.P.scheme == 50) sweeps<50>(a, s, st);
   else if (a.P.scheme == 71) sweeps<71>(a, s, st);
   else sweeps<51>(a, s, st);

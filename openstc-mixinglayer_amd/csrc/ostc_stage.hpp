@@ -15,7 +15,7 @@ struct StageBlock {
   int ntx, nty, tile_base, sp_jac;
   long long n0;
   gptr<const double> cvi, bvi, muli, qn, jac, met, sp_sigma, sp_mean;
-  gptr<double> cvo, bvo, mulo, mach, dq;
+  gptr<double> cvo, bvo, mulo, mach, dq, res;
 };
 
 __device__ __forceinline__ StageBlock stage_block(const DevBlock& B, int in, int out) {
@@ -36,6 +36,7 @@ __device__ __forceinline__ StageBlock stage_block(const DevBlock& B, int in, int
   S.mulo = (gptr<double>)B.mul[out];
   S.mach = (gptr<double>)B.mach;
   S.dq = (gptr<double>)B.dq;
+  S.res = (gptr<double>)B.res;
   return S;
 }
 
