@@ -561,21 +561,28 @@ void plain_rhs(const DevBlock& B, const Params& P, hipStream_t st, long long* n)
 }
 
 // Point kernels: 32 nodes along i, two whole 128-byte lines (with the (8,8,4)
-// of the reference half a line: 95x79x63 cells, the update 45 us, 23 us so).
-static const dim3 kPoints(32, 4, 2);
-static dim3 point_grid(int nx, int ny, int nz) {
-  return dim3((nx - 1) / kPoints.x + 1, (ny - 1) / kPoints.y + 1, (nz - 1) / kPoints.z + 1);
+// of the reference half a line: 95x79x63 cells, the update 45 us, 23 us so),
+// unless the block is so long that the grid would pass 65535 workgroups along y
+// or z: (8,8,4) has half as many.
+struct PointLaunch { dim3 grid, wg; };
+static PointLaunch point_launch(int nx, int ny, int nz) {
+  auto grid = [&](const dim3& w) { return dim3((nx - 1) / w.x + 1, (ny - 1) / w.y + 1, (nz - 1) / w.z + 1); };
+  dim3 wg(32, 4, 2);
+  if (grid(wg).y > 65535 || grid(wg).z > 65535) wg = dim3(8, 8, 4);
+  return PointLaunch{grid(wg), wg};
 }
-static dim3 interior_grid(const DevBlock& B) { return point_grid(B.mx, B.my, B.mz); }
+static PointLaunch interior(const DevBlock& B) { return point_launch(B.mx, B.my, B.mz); }
 
 void plain_update(const DevBlock& B, double dt, int rk, hipStream_t st, long long* n) {
   const RkCoef c = rk_coef(rk);
-  hipLaunchKernelGGL(k_update, interior_grid(B), kPoints, 0, st, B, dt, c.a, c.b, c.c);
+  const PointLaunch L = interior(B);
+  hipLaunchKernelGGL(k_update, L.grid, L.wg, 0, st, B, dt, c.a, c.b, c.c);
   *n += 1;
 }
 
 void plain_local_dt(const DevBlock& B, const Params& P, hipStream_t st, long long* n) {
-  hipLaunchKernelGGL(k_local_dt, interior_grid(B), kPoints, 0, st, B, P);
+  const PointLaunch L = interior(B);
+  hipLaunchKernelGGL(k_local_dt, L.grid, L.wg, 0, st, B, P);
   *n += 1;
 }
 
@@ -587,8 +594,8 @@ void min_reduce(const double* in, long long len, double* scratch, int n_first, h
 }
 
 void padded_pass(const DevBlock& B, int slot, int what, hipStream_t st, long long* n) {
-  const dim3 g = point_grid(B.mx + 2 * B.g, B.my + 2 * B.g, B.mz + 2 * B.g);
-  hipLaunchKernelGGL(k_padded, g, kPoints, 0, st, B, slot, what);
+  const PointLaunch L = point_launch(B.mx + 2 * B.g, B.my + 2 * B.g, B.mz + 2 * B.g);
+  hipLaunchKernelGGL(k_padded, L.grid, L.wg, 0, st, B, slot, what);
   *n += 1;
 }
 
