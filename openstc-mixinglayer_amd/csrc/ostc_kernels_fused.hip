@@ -730,8 +730,13 @@ void dt_rows(const FusedArgs& a, int n_blocks, long long max_cells, int n_wg, do
   const long long nx = std::min<long long>((max_cells + 255) / 256, std::max(1, n_wg / n_blocks));
   auto* bits = reinterpret_cast<unsigned long long*>(dt_bits);
   hipLaunchKernelGGL(k_dt_init, dim3(1), dim3(1), 0, st, bits);
-  hipLaunchKernelGGL(k_dt_rows, dim3((unsigned)nx, n_blocks), dim3(256), 0, st, a, bits);
-  *n += 2;
+  ++*n;
+  for (int first = 0; first < n_blocks; first += 65535) {  // most workgroups along y of a launch
+    FusedArgs some = a;
+    some.blocks += first;
+    hipLaunchKernelGGL(k_dt_rows, dim3((unsigned)nx, std::min(65535, n_blocks - first)), dim3(256), 0, st, some, bits);
+    ++*n;
+  }
 }
 
 }  // namespace ostc
