@@ -58,10 +58,9 @@ struct TileShape { int tx, ty, tz, waves_per_eu; };  // waves_per_eu: occupancy 
 int fused_shape_count(int scheme);
 TileShape fused_shape(int scheme, int index);
 // Launches the tile kernels of table entry `index`; mode 0 = RK update,
-// mode 1 = write dq only, mode 2 = RK update with the inviscid part of a
-// characteristic scheme in a kernel of its own.  The component-wise schemes'
-// inviscid dq is in place already (sweep_launch).  Returns the dynamic LDS
-// bytes used, or -1.
+// mode 1 = write dq only, mode 2 = RK update with the inviscid part in a kernel
+// of its own.  Returns the dynamic LDS bytes used, or -1 (not a characteristic
+// scheme, or a tile too large).
 int fused_launch(int index, int mode, const FusedArgs& a, int n_wg, hipStream_t st);
 int fused_lds_bytes(int scheme, int index);
 // Work list of the inviscid sweeps (ostc_kernels_sweep.hip).  x: one workgroup

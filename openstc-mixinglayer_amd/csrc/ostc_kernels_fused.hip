@@ -1,13 +1,14 @@
 // ostc_kernels_fused.hip -- the tile kernels of a batched RK stage over the
-// tiles of every block.  k_visc_update: second-order viscous fluxes staged
-// through LDS, added to the stored inviscid residual (ostc_kernels_sweep.hip
-// for the component-wise WENO schemes), then the SSP-RK3 update, primitives
-// and Sutherland viscosity.  k_fused: the characteristic WENO schemes (52,
-// 72) in one launch, their inviscid fluxes along x, y, z staged through LDS
-// and dq kept in registers (with the sponge layer's relaxation term first
-// where a block has one).  Both read ring slot `in` (state incl. ghosts) and
-// qn = slot 0 and write the interior of slot `out`; ghost layers are filled
-// afterwards by the op launches.
+// tiles of every block, for the characteristic WENO schemes (52, 72).  k_fused:
+// the whole stage in one launch, inviscid fluxes along x, y, z and second-order
+// viscous fluxes staged through LDS and dq kept in registers (with the sponge
+// layer's relaxation term first where a block has one), then the SSP-RK3 update,
+// primitives and Sutherland viscosity; or the inviscid part alone, its dq
+// stored, and k_visc_update for the rest (split stage).  Both read ring slot
+// `in` (state incl. ghosts) and qn = slot 0 and write the interior of slot `out`;
+// ghost layers are filled afterwards by the op launches.  The component-wise
+// schemes have kernels of their own (ostc_kernels_sweep.hip).  k_dt_rows, the
+// time step's minimum, serves all of them.
 //
 // Work decomposition: a tile is TX x TY x TZ cells of one block, one thread
 // per cell in the cell phases.  Each inviscid direction phase of k_fused
@@ -501,9 +502,8 @@ __device__ __forceinline__ void stage_update(const FusedArgs& A, const StageBloc
   B.mach[p] = sqrt(V2) / sqrt(c_temp * T);
 }
 
-// Viscous fluxes (VISC) and the RK update, starting from the stored inviscid
-// dq; UPDATE false: the viscous fluxes are added to the stored dq instead.
-template <int TX, int TY, int TZ, int WPE, int VISC, bool UPDATE>
+// Viscous fluxes and the RK update, starting from the stored inviscid dq.
+template <int TX, int TY, int TZ, int WPE>
 __global__ __launch_bounds__(TX * TY * TZ) __attribute__((amdgpu_waves_per_eu(WPE))) void k_visc_update(FusedArgs A) {
   extern __shared__ double smem[];
   TileCtx t;
@@ -519,14 +519,8 @@ __global__ __launch_bounds__(TX * TY * TZ) __attribute__((amdgpu_waves_per_eu(WP
 #pragma unroll
       for (int l = 0; l < 5; ++l) dq[l] = B.dq[q0 + l * n0];
     }
-    if (VISC) viscous_phase<TX, TY, TZ, ViscLds<TX, TY, TZ, WPE>::VSPLIT>(smem, B, A.P, t, dq);
-    if (!t.valid) continue;
-    if constexpr (UPDATE) {
-      stage_update(A, B, i, j, k, dq);
-    } else {
-#pragma unroll
-      for (int l = 0; l < 5; ++l) B.dq[q0 + l * n0] = dq[l];
-    }
+    viscous_phase<TX, TY, TZ, ViscLds<TX, TY, TZ, WPE>::VSPLIT>(smem, B, A.P, t, dq);
+    if (t.valid) stage_update(A, B, i, j, k, dq);
   }
 }
 
@@ -645,30 +639,14 @@ static void allow_lds(K kernel, int bytes) {
   (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
 }
 
-template <int TX, int TY, int TZ, int WPE>
-static void launch_visc(bool update, const FusedArgs& a, int n_wg, hipStream_t st) {
-  constexpr int bytes = ViscLds<TX, TY, TZ, WPE>::BYTES;
-  static bool attr_set = false;
-  if (bytes > 64 * 1024 && !attr_set) {
-    allow_lds(&k_visc_update<TX, TY, TZ, WPE, 1, true>, bytes);
-    allow_lds(&k_visc_update<TX, TY, TZ, WPE, 1, false>, bytes);
-    attr_set = true;
-  }
-  const dim3 grid(n_wg), block(TX * TY * TZ);
-  if (!a.P.visc) {
-    if (update) hipLaunchKernelGGL((k_visc_update<TX, TY, TZ, WPE, 0, true>), grid, block, 0, st, a);
-    return;
-  }
-  if (update) hipLaunchKernelGGL((k_visc_update<TX, TY, TZ, WPE, 1, true>), grid, block, bytes, st, a);
-  else hipLaunchKernelGGL((k_visc_update<TX, TY, TZ, WPE, 1, false>), grid, block, bytes, st, a);
-}
-
 template <int TX, int TY, int TZ, int WPE, int SCHEME>
 static int launch_shape(int mode, const FusedArgs& a, int n_wg, hipStream_t st) {
   constexpr int bytes = FusedLds<TX, TY, TZ, SCHEME, WPE>::BYTES;
+  constexpr int visc_bytes = ViscLds<TX, TY, TZ, WPE>::BYTES;
   if (bytes > 160 * 1024) return -1;
   static bool attr_set = false;
   if (!attr_set) {
+    allow_lds(&k_visc_update<TX, TY, TZ, WPE>, visc_bytes);
     allow_lds(&k_fused<TX, TY, TZ, WPE, SCHEME, 1, true>, bytes);
     allow_lds(&k_fused<TX, TY, TZ, WPE, SCHEME, 0, true>, bytes);
     allow_lds(&k_fused<TX, TY, TZ, WPE, SCHEME, 1, false>, bytes);
@@ -678,7 +656,7 @@ static int launch_shape(int mode, const FusedArgs& a, int n_wg, hipStream_t st) 
   const dim3 grid(n_wg), block(TX * TY * TZ);
   if (mode == 2 && a.P.visc) {  // split stage
     hipLaunchKernelGGL((k_fused<TX, TY, TZ, WPE, SCHEME, 0, false>), grid, block, bytes, st, a);
-    launch_visc<TX, TY, TZ, WPE>(true, a, n_wg, st);
+    hipLaunchKernelGGL((k_visc_update<TX, TY, TZ, WPE>), grid, block, visc_bytes, st, a);
     return bytes;
   }
   if (mode == 2) mode = 0;
@@ -692,9 +670,6 @@ static int launch_shape(int mode, const FusedArgs& a, int n_wg, hipStream_t st) 
 template <int TX, int TY, int TZ, int WPE>
 static int launch_scheme(int mode, const FusedArgs& a, int n_wg, hipStream_t st) {
   switch (a.P.scheme) {
-    case 50:
-    case 51:
-    case 71: launch_visc<TX, TY, TZ, WPE>(mode != 1, a, n_wg, st); return ViscLds<TX, TY, TZ, WPE>::BYTES;
     case 52: return launch_shape<TX, TY, TZ, WPE, 52>(mode, a, n_wg, st);
     case 72: return launch_shape<TX, TY, TZ, WPE, 72>(mode, a, n_wg, st);
     default: return -1;
