@@ -339,7 +339,8 @@ int ostc_residual(ostc_ctx ctx, double res[4]);
  * followed by a viscous + update kernel.  ostc_autotune times every
  * combination on the current blocks and keeps the fastest.  The sweeps of
  * schemes 50, 51 and 71 have no tile: for them the configuration is kept and
- * reported but changes nothing. */
+ * reported but changes nothing, and ostc_autotune times the stage and leaves it
+ * as it is. */
 int ostc_tile_count(int* n);
 int ostc_tile_shape(int index, int* tx, int* ty, int* tz);
 int ostc_set_tile(ostc_ctx ctx, int index, int waves_per_cu, int split);

@@ -1702,33 +1702,40 @@ int ostc_autotune(ostc_ctx c, int reps, int* best_index, double* best_ms) {
   if (r) return r;
   if ((r = need_fused(c)) || (r = need_residual(c))) return r;
   if (reps < 1) reps = 3;
-  double best = 1e30;
+  // ms per stage with the current configuration; negative: no kernel for it
+  auto time_stage = [&](double* ms) -> int {
+    long long n = 0;
+    FusedArgs a = fused_args(c, 0, 1, 0);
+    const int mode = c->split ? 2 : 0;
+    *ms = -1;
+    if (!launch_stage(c, mode, a, &n)) return OSTC_OK;  // warm-up
+    HIPCHK(c, hipEventRecord(c->ev_a, c->st));
+    for (int q = 0; q < reps; ++q) launch_stage(c, mode, a, &n);
+    HIPCHK(c, hipEventRecord(c->ev_b, c->st));
+    HIPCHK(c, hipEventSynchronize(c->ev_b));
+    HIPCHK(c, hipGetLastError());
+    float f = 0;
+    HIPCHK(c, hipEventElapsedTime(&f, c->ev_a, c->ev_b));
+    *ms = f / reps;
+    return OSTC_OK;
+  };
+  double best = 1e30, ms = 0;
   int bi = c->tile_index, bw = 0, bs = 0;
-  long long n = 0;
-  const int waves[] = {0, 1, 2, 4};
-  for (int idx = 0; idx < fused_shape_count(c->P.scheme); ++idx) {
-    const int lds = fused_lds_bytes(c->P.scheme, idx);
-    if (lds < 0 || lds > 160 * 1024) continue;
-    for (int sp = 0; sp < (c->P.visc && !sweep_scheme(c->P.scheme) ? 2 : 1); ++sp)
-      for (int w : waves) {
-        r = ostc_set_tile(c, idx, w, sp);
-        if (r) return r;
-        FusedArgs a = fused_args(c, 0, 1, 0);
-        const int mode = sp ? 2 : 0;
-        if (!launch_stage(c, mode, a, &n)) continue;  // warm-up
-        HIPCHK(c, hipEventRecord(c->ev_a, c->st));
-        for (int q = 0; q < reps; ++q) launch_stage(c, mode, a, &n);
-        HIPCHK(c, hipEventRecord(c->ev_b, c->st));
-        HIPCHK(c, hipEventSynchronize(c->ev_b));
-        HIPCHK(c, hipGetLastError());
-        float f = 0;
-        HIPCHK(c, hipEventElapsedTime(&f, c->ev_a, c->ev_b));
-        const double ms = f / reps;
-        if (ms < best) { best = ms; bi = idx; bw = w; bs = sp; }
-      }
+  if (sweep_scheme(c->P.scheme)) {  // nothing to choose: the configuration stays as it is
+    if ((r = time_stage(&best))) return r;
+  } else {
+    const int waves[] = {0, 1, 2, 4};
+    for (int idx = 0; idx < fused_shape_count(c->P.scheme); ++idx) {
+      const int lds = fused_lds_bytes(c->P.scheme, idx);
+      if (lds < 0 || lds > 160 * 1024) continue;
+      for (int sp = 0; sp < (c->P.visc ? 2 : 1); ++sp)
+        for (int w : waves) {
+          if ((r = ostc_set_tile(c, idx, w, sp)) || (r = time_stage(&ms))) return r;
+          if (ms >= 0 && ms < best) { best = ms; bi = idx; bw = w; bs = sp; }
+        }
+    }
+    if ((r = ostc_set_tile(c, bi, bw, bs))) return r;
   }
-  r = ostc_set_tile(c, bi, bw, bs);
-  if (r) return r;
   if (best_index) *best_index = bi;
   if (best_ms) *best_ms = best;
   return OSTC_OK;

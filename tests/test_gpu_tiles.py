@@ -72,3 +72,27 @@ def test_the_sweeps_have_no_tile():
     _, got, _ = _steps(case, 4, 2, 1)
     for x, y in zip(want, got):
         np.testing.assert_array_equal(x, y)
+
+
+def test_autotune_leaves_the_sweeps_configuration_alone():
+    print("[gpu] autotune of scheme 51", flush=True)
+    s = pkg.Solver(cases.small_multiblock_case())
+    s.setup_mixing_layer()
+    s.initialize()
+    for config in ((4, 2, 1), (1, 0, 0), (3, 4, 0)):
+        s.set_tile(*config)
+        index, ms = s.autotune(2)
+        assert index == config[0] and 0 < ms < 1e3
+        assert s.tile_config() == config
+    s.close()
+
+
+def test_autotune_of_a_characteristic_scheme():
+    print("[gpu] autotune of scheme 52", flush=True)
+    s = pkg.Solver(cases.small_multiblock_case(scheme=52))
+    s.setup_mixing_layer()
+    s.initialize()
+    index, ms = s.autotune(2)
+    assert 0 <= index < 6 and 0 < ms < 1e3
+    assert s.tile_config()[0] == index
+    s.close()
