@@ -14,7 +14,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("scheme", [50, 51, 71])
-@pytest.mark.parametrize("cells", [([33], [29], [31]), ([7, 9], [10], [8, 12])], ids=["one", "four"])
+@pytest.mark.parametrize("cells", [([33], [29], [31]), ([7, 9], [10], [8, 12]), ([6], [5], [6]),
+                                   ([5], [6], [135])], ids=["one", "four", "six", "long"])
 def test_inviscid_step_has_the_per_block_bits(cells, scheme):
     case = cases.mixing_layer_case(*cells, scheme=scheme, viscous_order=0, perturbation=2e-2)
     print(f"[gpu] batched rounding {cells} scheme {scheme}", flush=True)
