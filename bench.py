@@ -5,7 +5,7 @@ sizes (4 x 3 x 2 tensor-product cuts of 16..192 x 16..128 x 16..64 cells),
 about 12.5 M cells,
 WENO-Z5 component-wise + Lax-Friedrichs splitting, second-order viscous
 fluxes, SSP-RK3 at CFL 0.5, in-GPU inner-face exchange.  The BATCHED path
-(fused RHS+update kernel over the block work-list, graph-captured steps) is
+(each stage's RHS+update kernels over the blocks' work-lists) is
 the measured value; the PLAIN path (per-block launches shaped like the
 reference) is timed on the same state beside it.
 
@@ -310,9 +310,8 @@ def reacting_cpu_baseline(tables, n, steps, spatial=False):
 def measured_traffic():
     """HBM bytes of one stage's kernels (x sweep, y and z marches, viscous +
     update) on the 24-block case, from the FETCH_SIZE / WRITE_SIZE counter runs
-    summarised in profiles/fused_rhs_update_batched24_pmc.txt, or None."""
-    path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "profiles",
-                        "fused_rhs_update_batched24_pmc.txt")
+    summarised in profiles/batched24_pmc.txt, or None."""
+    path = os.path.join(ROOT, "profiles", "batched24_pmc.txt")
     if not os.path.exists(path):
         return None
     with open(path) as f:
@@ -336,12 +335,12 @@ def flop_counts(path=os.path.join(ROOT, "profiles", "flops_per_cell_air.txt")):
     return out
 
 
-def fused_roofline(cells, avg_kernel_ms, rate_mcells, tile_index, tile_split, tile_waves):
-    """Roofline of the fused RHS+update kernel (one RK stage over all blocks)
-    and of the whole step.  The kernel is measured against both roofs: HBM
-    with the contract-minimal 264 B per cell and stage, FP64 with the
-    oracle-counted flops per cell and stage; `bound` is the roof that binds
-    (the lower attainable rate), `achieved`/`peak`/`frac` are on that roof.
+def stage_roofline(cells, avg_kernel_ms, rate_mcells):
+    """Roofline of the RHS+update kernels of one RK stage over all blocks,
+    taken as one launch, and of the whole step.  They are measured against
+    both roofs: HBM with the contract-minimal 264 B per cell and stage, FP64
+    with the oracle-counted flops per cell and stage; `bound` is the roof that
+    binds (the lower attainable rate), `achieved`/`peak`/`frac` are on that roof.
     step: rate / min(8e12 / B_step, P_FP64 / F_step) in cell-updates/s."""
     f = flop_counts()
     avg_s = avg_kernel_ms / 1e3
@@ -358,8 +357,8 @@ def fused_roofline(cells, avg_kernel_ms, rate_mcells, tile_index, tile_split, ti
     fp64 = {"achieved": tfs, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": tfs / FP64_PEAK_TFLOPS}
     main = hbm if hbm_bound else fp64
     return {"bound": "hbm" if hbm_bound else "fp64", **main, "traffic": traffic,
-            "traffic_source": "profiles/fused_rhs_update_batched24_pmc.txt (rocprofv3 FETCH_SIZE + WRITE_SIZE, "
-                              "copy-calibrated, bytes per launch)" if traffic else None,
+            "traffic_source": "profiles/batched24_pmc.txt (rocprofv3 FETCH_SIZE + WRITE_SIZE, "
+                              "copy-calibrated, bytes per stage)" if traffic else None,
             "kernel": "k_sweep_x, k_sweep_march<1|2>, k_visc_update_rows (RHS+update, one RK stage over all blocks)",
             "hbm": hbm, "fp64": fp64,
             "algorithmic_bytes_per_launch": bytes_per_launch, "algorithmic_flops_per_launch": flops_per_launch,
@@ -394,9 +393,6 @@ def main():
     ap.add_argument("--plain-steps", type=int, default=20)
     ap.add_argument("--cpu-steps", type=int, default=2)
     ap.add_argument("--no-cpu", action="store_true")
-    ap.add_argument("--no-tune", action="store_true")
-    ap.add_argument("--tile", type=int, default=-1, metavar="INDEX",
-                    help="use this entry of the tile table (one workgroup per tile) instead of the autotuner")
     ap.add_argument("--no-adjoint", action="store_true")
     ap.add_argument("--no-characteristic", action="store_true", help="skip the scheme-52 batched/per-block leg")
     ap.add_argument("--adjoint-n", type=int, default=128)
@@ -435,18 +431,10 @@ def main():
     s = pkg.Solver(case)
     s.setup_mixing_layer()
     s.initialize()
-    if a.tile >= 0:
-        s.set_tile(a.tile, 0, 0)
-    elif not a.no_tune:
-        best = s.autotune(3)
-        print(f"[bench] autotune: best {best[1]:.3f} ms/stage", file=sys.stderr, flush=True)
-    tile_index, tile_waves, tile_split = s.tile_config()
-    print(f"[bench] fused kernel config: tile {pkg.tile_shapes()[tile_index]}, "
-          f"{tile_waves} workgroups/CU (0 = one per tile), split={tile_split}", file=sys.stderr, flush=True)
 
     # BATCHED: warm-up, then exactly K steps.  The timed region launches the
-    # batched kernels directly with HIP events around every fused RHS+update
-    # launch (the kernel durations behind the roofline figure); the same
+    # batched kernels directly with HIP events around every stage's RHS+update
+    # kernels (the durations behind the roofline figure); the same
     # steps replayed as a captured graph are timed afterwards as value_graph.
     s.rk3(a.warmup, pkg.MODE_BATCHED)
     s.sync()
@@ -458,7 +446,7 @@ def main():
     avg_kernel_ms, max_kernel_ms, n_kernel = s.fused_kernel_ms()
     value = cells * a.steps / wall / 1e6
     print(f"[bench] batched: {wall * 1e3 / a.steps:.3f} ms/step wall, {dev_ms / a.steps:.3f} ms/step device, "
-          f"fused kernel avg {avg_kernel_ms:.3f} ms max {max_kernel_ms:.3f} ms over {n_kernel} launches, "
+          f"RHS+update avg {avg_kernel_ms:.3f} ms max {max_kernel_ms:.3f} ms over {n_kernel} stages, "
           f"{launches // max(a.steps, 1)} launches/step", file=sys.stderr, flush=True)
     s.sync()
     t0 = time.perf_counter()
@@ -480,7 +468,7 @@ def main():
     print(f"[bench] plain: {wall_p * 1e3 / a.plain_steps:.3f} ms/step, "
           f"{launches_p // max(a.plain_steps, 1)} launches/step", file=sys.stderr, flush=True)
 
-    roofline = fused_roofline(cells, avg_kernel_ms, value, tile_index, tile_split, tile_waves)
+    roofline = stage_roofline(cells, avg_kernel_ms, value)
     s.close()
 
     characteristic = None if a.no_characteristic else characteristic_leg(5)
@@ -516,10 +504,7 @@ def main():
         "config": {"workload": f"batched multi-block air temporal mixing layer, 24 uneven blocks (cuts of 16..192 x "
                                f"16..128 x 16..64 cells, seed {pkg.cases.batched_seed()}), "
                                "WENO-Z5 cp + LF, 2nd-order viscous, SSP-RK3 CFL 0.5",
-                   "cells": cells, "blocks": len(case["blocks"]), "mode": "BATCHED",
-                   "tile": list(pkg.tile_shapes()[tile_index]), "tile_index": tile_index,
-                   "workgroups_per_cu": tile_waves,
-                   "split_stage": bool(tile_split)},
+                   "cells": cells, "blocks": len(case["blocks"]), "mode": "BATCHED"},
         "value_graph": value_graph, "plain_value": plain_value, "speedup_vs_plain": value / plain_value,
         "roofline": roofline, "cpu_baseline": cpu, "characteristic": characteristic, "adjoint": adjoint,
         "reacting": reacting, "parallel_faces": parallel,
