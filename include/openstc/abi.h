@@ -45,9 +45,9 @@ extern "C" {
 
 /* time-step modes of ostc_step */
 #define OSTC_MODE_PLAIN 0    /* per-block launches shaped like the reference */
-#define OSTC_MODE_BATCHED 1  /* fused RHS+update over a block work-list, graph-captured */
+#define OSTC_MODE_BATCHED 1  /* RHS+update over work-lists of every block, graph-captured */
 #define OSTC_MODE_BATCHED_TIMED 2  /* the batched kernels launched directly, with HIP events
-                                      around every fused launch (ostc_fused_kernel_ms) */
+                                      around every stage's RHS+update (ostc_fused_kernel_ms) */
 
 /* properties of the ghost layers after a batched stage (ostc_set_ghost_props) */
 #define OSTC_GHOST_PROPS_IN_OPS 0  /* each ghost op recomputes the nodes it writes (default) */
@@ -350,9 +350,9 @@ int ostc_autotune(ostc_ctx ctx, int reps, int* best_index, double* best_ms);
 /* Device timing of the last ostc_step call: total milliseconds measured
  * with HIP events on the context's stream, and the launch count. */
 int ostc_last_step_timing(ostc_ctx ctx, double* ms, long long* launches);
-/* Average and maximum duration (ms) of the fused RHS+update kernel over the
- * launches of the last OSTC_MODE_BATCHED_TIMED ostc_step call, from HIP
- * events recorded around each launch on the context's stream. */
+/* Average and maximum duration (ms) of a stage's RHS+update kernels over the
+ * stages of the last OSTC_MODE_BATCHED_TIMED ostc_step call, from HIP
+ * events recorded around each stage's on the context's stream. */
 int ostc_fused_kernel_ms(ostc_ctx ctx, double* avg_ms, double* max_ms, long long* count);
 int ostc_sync(ostc_ctx ctx);
 const char* ostc_last_error(ostc_ctx ctx);

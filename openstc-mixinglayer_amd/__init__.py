@@ -537,7 +537,7 @@ class Solver:
         return ms.value, n.value
 
     def fused_kernel_ms(self):
-        """(average ms, max ms, launches) of the fused kernel in the last timed step call."""
+        """(average ms, max ms, stages) of a stage's RHS+update kernels in the last timed step call."""
         avg, mx, n = C.c_double(), C.c_double(), C.c_longlong()
         self._chk(lib().ostc_fused_kernel_ms(self.ctx, C.byref(avg), C.byref(mx), C.byref(n)))
         return avg.value, mx.value, n.value

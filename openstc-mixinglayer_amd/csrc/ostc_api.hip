@@ -124,7 +124,7 @@ struct ostc_ctx_s {
   hipGraph_t graph = nullptr;
   hipGraphExec_t gexec = nullptr;
   bool graph_valid = false;
-  std::vector<hipEvent_t> evpool;  // pairs around fused launches (timed mode)
+  std::vector<hipEvent_t> evpool;  // pairs around a stage's RHS + update (timed mode)
   long long timed_launches = 0;
   hipEvent_t ev_a = nullptr, ev_b = nullptr;
   long long graph_launches = 0;
@@ -518,8 +518,8 @@ int upload_blocks(ostc_ctx c) {
   return OSTC_OK;
 }
 
-// The fused batched kernel and the reverse mode implement the component-wise
-// WENO schemes 50/51/71 and the characteristic WENO-Z 52/72; the primitive
+// The batched kernels implement the component-wise WENO schemes 50/51/71 and
+// the characteristic WENO-Z 52/72 (the reverse mode 50 and 51); the primitive
 // reconstruction + Riemann schemes (1/2/3/4) and EP6 run on the per-block kernels.
 bool fused_scheme(const ostc_ctx c) {
   const int sc = c->P.scheme;
@@ -527,7 +527,7 @@ bool fused_scheme(const ostc_ctx c) {
 }
 
 int need_fused(ostc_ctx c) {
-  for (auto& B : c->blocks)  // the fused kernel indexes a block's planes with 32-bit offsets
+  for (auto& B : c->blocks)  // the batched kernels index a block's planes with 32-bit offsets
     if (9 * B.d.sz >= (1LL << 31))
       return fail(c, OSTC_ERR_UNSUPPORTED, "block too large for the batched kernel (9 padded planes >= 2^31 doubles)");
   if (fused_scheme(c)) return OSTC_OK;
@@ -808,11 +808,9 @@ int dual_step(ostc_ctx c, long long* n) {
 }
 
 // ------------------------------------------------------- batched step
-// One batched step.  ev_base >= 0: record event pairs evpool[ev_base + 2 rk],
-// evpool[ev_base + 2 rk + 1] around the fused kernel of stage rk.
 // Stage rk of a batched step: ring slot rk -> slot (rk+1) % 3, then the
 // ghost layers of the new slot.  ev_base >= 0: events evpool[ev_base + 2 rk],
-// evpool[ev_base + 2 rk + 1] around the fused kernel.
+// evpool[ev_base + 2 rk + 1] around its RHS + update kernels.
 int batched_stage(ostc_ctx c, int rk, long long* n, int ev_base) {
   const bool events = ev_base >= 0;
   const int in = rk, out = (rk + 1) % kRing;

@@ -40,7 +40,7 @@ void dual_update(const DevBlock& B, hipStream_t st, long long* n);
 void dual_last_store(const DevBlock& B, const DualBlock& D, hipStream_t st);
 void dual_last_square(const DevBlock& B, const DualBlock& D, double* out4, int nblk, hipStream_t st);
 
-// fused multi-block path, ostc_kernels_fused.hip
+// batched path, ostc_kernels_sweep.hip and ostc_kernels_fused.hip
 struct FusedArgs {
   const DevBlock* blocks;
   const int* tile_block;     // block of each tile

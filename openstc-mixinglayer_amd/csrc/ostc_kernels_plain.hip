@@ -3,7 +3,7 @@
 // and viscous fluxes with dq read-modify-write in HBM, a point kernel each for
 // the update and the local time step, a two-pass MIN with a host read-back for
 // dt, and launches per block or inner face for the ghost layers.  This is
-// the drop-in path; the fused batched kernel lives in ostc_kernels_fused.hip.
+// the drop-in path; the batched kernels live in ostc_kernels_sweep.hip and ostc_kernels_fused.hip.
 #include "ostc_kernels.hpp"
 
 namespace ostc {

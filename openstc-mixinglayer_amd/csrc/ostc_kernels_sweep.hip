@@ -13,9 +13,10 @@
 // a point evaluated 6.4 times, a third of its instructions spent on indexes.
 // Here a wave depends on no other wave.  The price is dq, stored and read
 // between the kernels (0.3 KB a node and stage).  Measured on the same case:
-// x sweep 0.43 ms, y 0.60, z 0.56, viscous + update 1.42 (6.7 GB, 4.7 TB/s),
-// the step 14.4 -> 10.1 ms; 16^3 nodes 114 -> 111 us; 101x75x49 nodes with
-// WENO-Z7 603 -> 495 us.
+// x sweep 0.43 ms (4.1 TB/s), y 0.59 (5.0), z 0.55 (5.2), viscous + update 1.40
+// (6.9 GB, 4.9 TB/s); when they took the tile kernel's place the step went from
+// 14.4 to 10.1 ms (10.2 in the present rounding), 16^3 nodes from 114 to 111 us,
+// 101x75x49 nodes with WENO-Z7 from 603 to 495 us.
 #include "ostc_stage.hpp"
 
 namespace ostc {

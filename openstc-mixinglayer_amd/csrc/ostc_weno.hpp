@@ -21,9 +21,11 @@
 // being one estimate and three FMAs.
 // By itself, in the tile kernels that then did every scheme: a step of 24 air
 // blocks (12.5 M nodes, WENO-Z5) 16.25 -> 14.42 ms, WENO-Z7 on 101x75x49 nodes
-// 688 -> 603 us, characteristic 1.97 -> 1.78 ms, a reacting 256x128x64 block
-// 20.3 -> 19.5 ms.  The error of a step against 64-bit whole-array
-// arithmetic in another order is no larger (7.2e-15 -> 6.9e-15 of v on 16^3).
+// 688 -> 603 us, characteristic 1.91 -> 1.78 ms, a reacting 256x128x64 block
+// 20.3 -> 19.5 ms.  The error of a step against 64-bit whole-array arithmetic
+// in another order (mean of 6 seeds) is no larger: w on 16^3 nodes 6.85e-15 ->
+// 6.52e-15, on 64^3 (WENO5-JS) 5.38e-15 -> 5.04e-15, v on 101x75x49 (WENO-Z7)
+// 4.31e-14 -> 4.31e-14.
 #pragma once
 #include <hip/hip_runtime.h>
 
